@@ -499,6 +499,18 @@ int relm_mp_film_mish_backward(const float* s, const float* dy, int64_t rows, in
                                const float* beta, const float* add, float* ds, double* partial,
                                int64_t partial_blocks, relm_mp_stream_t stream);
 
+/* relm_mp_film_mish_backward with the block sums added up on the device: sums
+ * [num_ranges, 2, width] (float32) receives per range the gradients of gamma[k] and
+ * of beta[k] (zero for an empty range), added in fp64 and rounded once.  workspace:
+ * relm_mp_film_mish_backward_sums_workspace_size(...) bytes, 8-byte aligned. */
+size_t relm_mp_film_mish_backward_sums_workspace_size(const int64_t* range_start, int32_t num_ranges,
+                                                      int64_t width);
+int relm_mp_film_mish_backward_sums(const float* s, const float* dy, int64_t rows, int64_t width,
+                                    const int64_t* range_start, int32_t num_ranges,
+                                    const float* gamma, const float* beta, const float* add,
+                                    float* ds, float* sums, void* workspace, size_t workspace_bytes,
+                                    relm_mp_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

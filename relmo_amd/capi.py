@@ -69,6 +69,8 @@ EXPORTED_SYMBOLS = (
     "relm_mp_film_mish",
     "relm_mp_film_mish_blocks",
     "relm_mp_film_mish_backward",
+    "relm_mp_film_mish_backward_sums_workspace_size",
+    "relm_mp_film_mish_backward_sums",
 )
 
 
@@ -183,6 +185,9 @@ _SIGNATURES = {
     "relm_mp_film_mish_blocks": (_i64, [_vp, ctypes.c_int32]),
     "relm_mp_film_mish_backward": (
         _int, [_vp, _vp, _i64, _i64, _vp, ctypes.c_int32, _vp, _vp, _vp, _vp, _vp, _i64, _vp]),
+    "relm_mp_film_mish_backward_sums_workspace_size": (_sz, [_vp, ctypes.c_int32, _i64]),
+    "relm_mp_film_mish_backward_sums": (
+        _int, [_vp, _vp, _i64, _i64, _vp, ctypes.c_int32, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _vp]),
     "relm_mp_plan_match": (
         _int,
         [_vp, _vp, _i64, ctypes.POINTER(_PP), ctypes.c_int32, ctypes.POINTER(ctypes.c_int32), _vp,
@@ -698,6 +703,20 @@ def film_mish_backward(dy: torch.Tensor, s: torch.Tensor, range_start: list[int]
                                            _ptr(gamma), _ptr(beta), _ptr(add) if add is not None else None,
                                            _ptr(ds), _ptr(partial), blocks, _stream(s)))
     return ds, partial[:blocks]
+
+
+def film_mish_backward_sums(dy: torch.Tensor, s: torch.Tensor, range_start: list[int], gamma: torch.Tensor,
+                            beta: torch.Tensor, add: torch.Tensor | None = None):
+    """``relm_mp_film_mish_backward_sums``: (ds, column sums per range [ranges, 2, width], float32)."""
+
+    starts, k = _starts(range_start)
+    ws = _bytes(lib().relm_mp_film_mish_backward_sums_workspace_size(starts, k, s.size(1)), s)
+    ds = torch.empty_like(s)
+    sums = torch.empty(k, 2, s.size(1), dtype=torch.float32, device=s.device)
+    check(lib().relm_mp_film_mish_backward_sums(_ptr(s), _ptr(dy), s.size(0), s.size(1), starts, k,
+                                                _ptr(gamma), _ptr(beta), _ptr(add) if add is not None else None,
+                                                _ptr(ds), _ptr(sums), _ptr(ws), ws.numel(), _stream(s)))
+    return ds, sums
 
 
 def plan_match(keys: torch.Tensor, gathers: torch.Tensor | None, plans: list[BuiltPlan]) -> list[bool]:

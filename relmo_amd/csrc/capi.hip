@@ -725,6 +725,37 @@ int relm_mp_film_mish_backward(const float* s, const float* dy, int64_t rows, in
     return RELM_MP_OK;
 }
 
+size_t relm_mp_film_mish_backward_sums_workspace_size(const int64_t* range_start, int32_t num_ranges,
+                                                      int64_t width) {
+    if (num_ranges < 1 || num_ranges > kFilmMaxRanges || range_start == nullptr || width < 0) return 0;
+    return film_sums_workspace(range_start, num_ranges, width);
+}
+
+int relm_mp_film_mish_backward_sums(const float* s, const float* dy, int64_t rows, int64_t width,
+                                    const int64_t* range_start, int32_t num_ranges,
+                                    const float* gamma, const float* beta, const float* add,
+                                    float* ds, float* sums, void* workspace, size_t workspace_bytes,
+                                    relm_mp_stream_t stream) {
+    RELM_TRY(check_rows(rows, "rows"));
+    if (width < 0 || width > 0x7fffffff)
+        return set_error(RELM_MP_ERR_INVALID_ARGUMENT, "relm_mp film: width must be in [0, 2^31).");
+    RELM_TRY(check_film_ranges(range_start, num_ranges, rows));
+    if (width == 0) return RELM_MP_OK;
+    const size_t need = film_sums_workspace(range_start, num_ranges, width);
+    if (workspace_bytes < need || (need > 0 && workspace == nullptr))
+        return set_error(RELM_MP_ERR_WORKSPACE, "relm_mp film: workspace too small");
+    if (reinterpret_cast<uintptr_t>(workspace) % sizeof(double) != 0)
+        return set_error(RELM_MP_ERR_INVALID_ARGUMENT, "relm_mp film: workspace not 8-byte aligned");
+    if (sums == nullptr || (rows > 0 && (s == nullptr || dy == nullptr || gamma == nullptr ||
+                                         beta == nullptr || ds == nullptr)))
+        return set_error(RELM_MP_ERR_INVALID_ARGUMENT, "relm_mp film: NULL array");
+    RELM_HIP(launch_film_mish_backward_sums(s, dy, width, range_start, num_ranges, gamma, beta, add,
+                                            ds, sums, static_cast<double*>(workspace),
+                                            static_cast<hipStream_t>(stream)),
+             "relm_mp film backward kernels");
+    return RELM_MP_OK;
+}
+
 int relm_mp_pack_index(const relm_mp_index_part* parts, int32_t num_parts, int64_t* out_a,
                        int64_t* out_b, relm_mp_stream_t stream) {
     if (num_parts < 0 || (num_parts > 0 && parts == nullptr))

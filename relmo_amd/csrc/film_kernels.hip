@@ -11,8 +11,6 @@
 // gradients.
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
-
 #include "device_utils.h"
 #include "internal.h"
 
@@ -20,16 +18,17 @@ namespace relm_mp {
 
 namespace {
 
-constexpr int kMaxThreads = 1024;
+constexpr int kThreads = 256;
+constexpr int64_t kCus = 256;
 constexpr int kMaxRanges = RELM_MP_FILM_MAX_RANGES;
-constexpr int kRowsPerBlock = RELM_MP_FILM_ROWS_PER_BLOCK;
 
-// Range k covers rows [start[k], start[k + 1]); its blocks of kRowsPerBlock
-// rows are blocks [first_block[k], first_block[k + 1]) of the grid, so no
-// block spans two ranges.
+// Range k covers rows [start[k], start[k + 1]); its blocks of rows_per_block
+// rows are blocks [first_block[k], first_block[k + 1]), so no block spans two
+// ranges.
 struct FilmRanges {
     int64_t start[kMaxRanges + 1];
     int64_t first_block[kMaxRanges + 1];
+    int64_t rows_per_block;
     int num;
 };
 
@@ -68,222 +67,278 @@ __device__ __forceinline__ float mish_backward(float dy, float u) {
     return dy * fmaf(u * sg, fmaf(-t, t, 1.0f), t);
 }
 
+// V floats that start at any 4-byte aligned address: one 16-byte access for V =
+// 4 (global memory takes it at dword alignment), so rows of any width move in
+// 16-byte pieces.
 template <int V>
-using Vec = Pack<float, V>;
+using Vec = float __attribute__((ext_vector_type(V), aligned(4)));
 
-// The block's rows and its range: blocks of a range are consecutive.
+template <int V>
+__device__ __forceinline__ Vec<V> load(const float* p) {
+    return *reinterpret_cast<const Vec<V>*>(p);
+}
+template <int V>
+__device__ __forceinline__ Vec<V> load_stream(const float* p) {
+    return __builtin_nontemporal_load(reinterpret_cast<const Vec<V>*>(p));
+}
+template <int V>
+__device__ __forceinline__ void store_stream(float* p, Vec<V> x) {
+    __builtin_nontemporal_store(x, reinterpret_cast<Vec<V>*>(p));
+}
+
+// A workgroup's rows and their range: blocks of a range are consecutive.
 struct BlockRows {
     int k;
     int64_t r0;
     int64_t r1;
 };
 
-__device__ __forceinline__ BlockRows block_rows(const FilmRanges& R) {
-    const int64_t b = blockIdx.x;
+__device__ __forceinline__ BlockRows block_rows(const FilmRanges& R, int64_t b) {
     int k = 0;
 #pragma unroll
     for (int q = 1; q < kMaxRanges; ++q)
         if (q < R.num && b >= R.first_block[q]) k = q;
-    const int64_t r0 = R.start[k] + (b - R.first_block[k]) * kRowsPerBlock;
-    const int64_t r1 = min(r0 + kRowsPerBlock, R.start[k + 1]);
+    const int64_t r0 = R.start[k] + (b - R.first_block[k]) * R.rows_per_block;
+    const int64_t r1 = min(r0 + R.rows_per_block, R.start[k + 1]);
     return {k, r0, r1};
 }
 
-// Thread layout of both kernels: `phases` groups of `units` threads (one per
-// column unit of V floats); thread t owns unit t % units and, within the
-// workgroup's block of rows, the rows r0 + p, r0 + p + phases, ... (p = t /
-// units).  Several phases keep the lanes busy where a row has fewer units
-// than the workgroup threads (C5: 199 pairs of floats per row, 5 phases over
-// 1024 threads); with one phase the threads loop over the units instead (rows
-// wider than the workgroup).  A thread keeps its columns, so the backward's
-// column sums need no atomics.
+// Thread layout of both kernels.  The columns are units of V floats; where the
+// width is no multiple of V the last unit is shifted back to end with the row,
+// and the columns it shares with the unit before are computed twice with equal
+// results.  A workgroup takes `units` neighbouring units of one block of rows,
+// `phases` rows at a time: thread t owns unit t % units and the block's rows t /
+// units, t / units + phases, ...  A thread keeps its columns, so their tables
+// stay in registers and the backward's column sums need no atomics.
 struct FilmLayout {
-    int units;   // column units per row
-    int phases;  // row phases
+    int total;   // units of a row
+    int chunks;  // workgroups side by side over the columns
+    int units;   // units of one workgroup
+    int phases;  // rows of one workgroup at a time
+};
+
+struct FilmThread {
+    int64_t col;
+    int unit;
+    int phase;
+    bool active;
 };
 
 template <int V>
-__global__ __launch_bounds__(kMaxThreads) void k_film_mish(const float* __restrict__ s,
-                                                           int64_t width, FilmRanges R, FilmLayout L,
-                                                           const float* __restrict__ gamma,
-                                                           const float* __restrict__ beta,
-                                                           const float* __restrict__ add,
-                                                           float* __restrict__ y) {
-    const BlockRows br = block_rows(R);
+__device__ __forceinline__ FilmThread film_thread(const FilmLayout& L, int chunk, int64_t width) {
     const int t = static_cast<int>(threadIdx.x);
-    const int ph = L.phases > 1 ? t / L.units : 0;
-    if (ph >= L.phases) return;
-    const int step = L.phases;
-    for (int64_t c = L.phases > 1 ? t % L.units : t; c < L.units; c += L.phases > 1 ? L.units : blockDim.x) {
-        const int64_t col = c * V;
-        const Vec<V> g = pack_load<float, V>(gamma + br.k * width + col);
-        const Vec<V> b = pack_load<float, V>(beta + br.k * width + col);
-        const Vec<V> a = add != nullptr ? pack_load<float, V>(add + br.k * width + col)
-                                        : pack_fill<float, V>(0.0f);
-        int64_t r = br.r0 + ph;
-        for (; r + 3 * step < br.r1; r += 4 * step) {
-            Vec<V> x[4];
+    FilmThread f;
+    f.phase = t / L.units;
+    f.unit = t - f.phase * L.units;
+    const int u = chunk * L.units + f.unit;
+    f.active = f.phase < L.phases && u < L.total;
+    f.col = min(static_cast<int64_t>(u) * V, width - V);
+    return f;
+}
+
+// Rows a thread has in flight: the loads of kRows rows are issued before the
+// first of them is used.
+constexpr int kRows = 2;
+
+// Bound by the vector units, not by memory: about 125 lane instructions per
+// element, three quarters of them log1pf, so 400 M elements take 1.2 ms at any
+// split while moving them takes 0.64.  The workgroups are small (4 waves) and
+// many, so that the last ones leave few CUs idle: [1,000,003 x 400] takes 1.34
+// ms, [204,800 x 96] 76 us and [2,000 x 400] 10 us, against 1.46 ms, 86 us and
+// 158 us with 768 threads to a workgroup of 512 whole rows.
+template <int V>
+__global__ __launch_bounds__(kThreads) void k_film_mish(const float* __restrict__ s, int64_t width,
+                                                        FilmRanges R, FilmLayout L,
+                                                        const float* __restrict__ gamma,
+                                                        const float* __restrict__ beta,
+                                                        const float* __restrict__ add,
+                                                        float* __restrict__ y) {
+    const int chunk = static_cast<int>(blockIdx.x % L.chunks);
+    const BlockRows br = block_rows(R, blockIdx.x / L.chunks);
+    const FilmThread f = film_thread<V>(L, chunk, width);
+    if (!f.active) return;
+    const Vec<V> g = load<V>(gamma + br.k * width + f.col);
+    const Vec<V> b = load<V>(beta + br.k * width + f.col);
+    const Vec<V> a = add != nullptr ? load<V>(add + br.k * width + f.col) : Vec<V>(0.0f);
+    auto step = [&](const Vec<V>& x, int64_t r) {
+        Vec<V> o;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) x[j] = pack_load_stream<float, V>(s + (r + j * step) * width + col);
+        for (int i = 0; i < V; ++i) o[i] = mish(b[i] + g[i] * (x[i] + a[i]));
+        store_stream<V>(y + r * width + f.col, o);
+    };
+    int64_t r = br.r0 + f.phase;
+    for (; r + (kRows - 1) * L.phases < br.r1; r += kRows * L.phases) {
+        Vec<V> x[kRows];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                Vec<V> o;
+        for (int j = 0; j < kRows; ++j) x[j] = load_stream<V>(s + (r + j * L.phases) * width + f.col);
 #pragma unroll
-                for (int i = 0; i < V; ++i) o.v[i] = mish(b.v[i] + g.v[i] * (x[j].v[i] + a.v[i]));
-                pack_store_stream<float, V>(y + (r + j * step) * width + col, o);
-            }
-        }
-        for (; r < br.r1; r += step) {
-            const Vec<V> x = pack_load_stream<float, V>(s + r * width + col);
-            Vec<V> o;
-#pragma unroll
-            for (int i = 0; i < V; ++i) o.v[i] = mish(b.v[i] + g.v[i] * (x.v[i] + a.v[i]));
-            pack_store_stream<float, V>(y + r * width + col, o);
-        }
+        for (int j = 0; j < kRows; ++j) step(x[j], r + j * L.phases);
     }
+    for (; r < br.r1; r += L.phases) step(load_stream<V>(s + r * width + f.col), r);
 }
 
 // ds = dy * mish'(u) * gamma; partial[block][0][col] = sum over the block's
 // rows of du * (s + add), partial[block][1][col] = sum of du, du = dy *
 // mish'(u), each term rounded to fp32 and added in fp64: by each thread over
 // its rows in row order, then the phases in order.  The block sums stay fp64
-// (the caller adds a range's blocks in fp64 and rounds once), so a per-range
-// sum over tens of thousands of rows carries only the rounding of its terms.
-// With several phases, `lds` holds phases * units * V * 2 doubles.
+// (a range's blocks are added in fp64 and rounded once), so a per-range sum
+// over tens of thousands of rows carries only the rounding of its terms.
+// `lds` holds phases * units * V * 2 doubles.  Bound as the forward is: [1,000,003
+// x 400] takes 1.67 ms with the sums, [204,800 x 96] 101 us, against 2.18 ms and
+// 134 us with the forward's former split and torch's sums.
 template <int V>
-__global__ __launch_bounds__(kMaxThreads) void k_film_mish_backward(
+__global__ __launch_bounds__(kThreads) void k_film_mish_backward(
     const float* __restrict__ s, const float* __restrict__ dy, int64_t width, FilmRanges R,
     FilmLayout L, const float* __restrict__ gamma, const float* __restrict__ beta,
     const float* __restrict__ add, float* __restrict__ ds, double* __restrict__ partial) {
     extern __shared__ double lds[];
-    const BlockRows br = block_rows(R);
-    const int t = static_cast<int>(threadIdx.x);
-    const int ph = L.phases > 1 ? t / L.units : 0;
-    const int step = L.phases;
-    double* __restrict__ part = partial + static_cast<int64_t>(blockIdx.x) * 2 * width;
-    const bool active = ph < L.phases;
-    for (int64_t c = L.phases > 1 ? t % L.units : t; active && c < L.units;
-         c += L.phases > 1 ? L.units : blockDim.x) {
-        const int64_t col = c * V;
-        const Vec<V> g = pack_load<float, V>(gamma + br.k * width + col);
-        const Vec<V> b = pack_load<float, V>(beta + br.k * width + col);
-        const Vec<V> a = add != nullptr ? pack_load<float, V>(add + br.k * width + col)
-                                        : pack_fill<float, V>(0.0f);
+    const int chunk = static_cast<int>(blockIdx.x % L.chunks);
+    const int64_t block = blockIdx.x / L.chunks;
+    const BlockRows br = block_rows(R, block);
+    const FilmThread f = film_thread<V>(L, chunk, width);
+    if (f.active) {
+        const Vec<V> g = load<V>(gamma + br.k * width + f.col);
+        const Vec<V> b = load<V>(beta + br.k * width + f.col);
+        const Vec<V> a = add != nullptr ? load<V>(add + br.k * width + f.col) : Vec<V>(0.0f);
         double sum_t[V], sum_u[V];
 #pragma unroll
         for (int i = 0; i < V; ++i) sum_t[i] = sum_u[i] = 0.0;
-        auto stp = [&](const Vec<V>& x, const Vec<V>& d, int64_t r) {
+        auto step = [&](const Vec<V>& x, const Vec<V>& d, int64_t r) {
             Vec<V> o;
 #pragma unroll
             for (int i = 0; i < V; ++i) {
-                const float tt = x.v[i] + a.v[i];
-                const float du = mish_backward(d.v[i], b.v[i] + g.v[i] * tt);
-                o.v[i] = du * g.v[i];
+                const float tt = x[i] + a[i];
+                const float du = mish_backward(d[i], b[i] + g[i] * tt);
+                o[i] = du * g[i];
                 sum_t[i] += static_cast<double>(du * tt);
                 sum_u[i] += static_cast<double>(du);
             }
-            pack_store_stream<float, V>(ds + r * width + col, o);
+            store_stream<V>(ds + r * width + f.col, o);
         };
-        int64_t r = br.r0 + ph;
-        for (; r + 3 * step < br.r1; r += 4 * step) {
-            Vec<V> x[4], d[4];
+        int64_t r = br.r0 + f.phase;
+        for (; r + (kRows - 1) * L.phases < br.r1; r += kRows * L.phases) {
+            Vec<V> x[kRows], d[kRows];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                x[j] = pack_load_stream<float, V>(s + (r + j * step) * width + col);
-                d[j] = pack_load_stream<float, V>(dy + (r + j * step) * width + col);
+            for (int j = 0; j < kRows; ++j) {
+                x[j] = load_stream<V>(s + (r + j * L.phases) * width + f.col);
+                d[j] = load_stream<V>(dy + (r + j * L.phases) * width + f.col);
             }
 #pragma unroll
-            for (int j = 0; j < 4; ++j) stp(x[j], d[j], r + j * step);
+            for (int j = 0; j < kRows; ++j) step(x[j], d[j], r + j * L.phases);
         }
-        for (; r < br.r1; r += step)
-            stp(pack_load_stream<float, V>(s + r * width + col),
-                pack_load_stream<float, V>(dy + r * width + col), r);
-        if (L.phases > 1) {
-            // this thread's sums into LDS: [phase][unit][V] for t, then for u
-            double* lt = lds + (static_cast<int64_t>(ph) * L.units + c) * V;
-            double* lu = lt + static_cast<int64_t>(L.phases) * L.units * V;
+        for (; r < br.r1; r += L.phases)
+            step(load_stream<V>(s + r * width + f.col), load_stream<V>(dy + r * width + f.col), r);
+        // this thread's sums into LDS: [phase][t or u][unit][V]
+        double* l = lds + (static_cast<int64_t>(f.phase) * 2 * L.units + f.unit) * V;
 #pragma unroll
-            for (int i = 0; i < V; ++i) {
-                lt[i] = sum_t[i];
-                lu[i] = sum_u[i];
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < V; ++i) {
-                part[col + i] = sum_t[i];
-                part[width + col + i] = sum_u[i];
-            }
+        for (int i = 0; i < V; ++i) {
+            l[i] = sum_t[i];
+            l[L.units * V + i] = sum_u[i];
         }
     }
-    if (L.phases > 1) {
-        __syncthreads();
-        // phase 0's threads add the phases in order
-        if (active && ph == 0) {
-            const int c = t;
-            const int64_t col = static_cast<int64_t>(c) * V;
-#pragma unroll
-            for (int i = 0; i < V; ++i) {
-                double at = 0.0, au = 0.0;
-                for (int p = 0; p < L.phases; ++p) {
-                    const double* lt = lds + (static_cast<int64_t>(p) * L.units + c) * V;
-                    at += lt[i];
-                    au += lt[static_cast<int64_t>(L.phases) * L.units * V + i];
-                }
-                part[col + i] = at;
-                part[width + col + i] = au;
-            }
-        }
+    __syncthreads();
+    // one thread per (t or u, column) adds the phases in order
+    const int sums = 2 * L.units * V;
+    for (int i = static_cast<int>(threadIdx.x); i < sums; i += kThreads) {
+        const int which = i / (L.units * V), at = i - which * (L.units * V);
+        const int u = chunk * L.units + at / V;
+        if (u >= L.total) continue;
+        double sum = 0.0;
+        for (int p = 0; p < L.phases; ++p) sum += lds[static_cast<int64_t>(p) * sums + i];
+        const int64_t col = min(static_cast<int64_t>(u) * V, width - V) + at % V;
+        partial[(block * 2 + which) * width + col] = sum;
     }
 }
 
-// Floats per lane: 4 where the width and every table are 16-byte aligned,
-// else 2 where they are 8-byte aligned, else 1.
-int film_vec(int64_t width, std::initializer_list<const void*> ptrs) {
-    for (int v : {4, 2}) {
-        bool ok = width % v == 0;
-        for (const void* p : ptrs) ok = ok && (p == nullptr || reinterpret_cast<uintptr_t>(p) % (4 * v) == 0);
-        if (ok) return v;
+// sums[k][j] = sum over range k's blocks of partial[block][j] (j < 2 * width),
+// added in fp64 and rounded to fp32 once: kFoldCols columns by kFoldRows blocks
+// at a time, then the kFoldRows parts in order.  Latency bound (at most a few
+// tens of MB over many short chains): torch's sum took 16 us per range and a
+// copy each.
+constexpr int kFoldCols = 16;
+constexpr int kFoldRows = kThreads / kFoldCols;
+
+__global__ __launch_bounds__(kThreads) void k_film_fold(const double* __restrict__ partial, int64_t cols,
+                                                        FilmRanges R, float* __restrict__ sums) {
+    __shared__ double lds[kFoldRows][kFoldCols];
+    const int c = static_cast<int>(threadIdx.x) % kFoldCols, q = static_cast<int>(threadIdx.x) / kFoldCols;
+    const int k = static_cast<int>(blockIdx.y);
+    const int64_t j = static_cast<int64_t>(blockIdx.x) * kFoldCols + c;
+    double sum = 0.0;
+    if (j < cols) {
+        const int64_t b1 = R.first_block[k + 1];
+        int64_t b = R.first_block[k] + q;
+        for (; b + 3 * kFoldRows < b1; b += 4 * kFoldRows) {
+            double v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = partial[(b + i * kFoldRows) * cols + j];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sum += v[i];
+        }
+        for (; b < b1; b += kFoldRows) sum += partial[b * cols + j];
     }
-    return 1;
+    lds[q][c] = sum;
+    __syncthreads();
+    if (q == 0 && j < cols) {
+        for (int i = 1; i < kFoldRows; ++i) sum += lds[i][c];
+        sums[k * cols + j] = static_cast<float>(sum);
+    }
 }
 
-FilmRanges film_ranges(const int64_t* range_start, int32_t num_ranges) {
+FilmRanges film_ranges(const int64_t* range_start, int32_t num_ranges, int64_t rows_per_block) {
     FilmRanges R{};
     int64_t blocks = 0;
     for (int k = 0; k < num_ranges; ++k) {
         R.start[k] = range_start[k];
         R.first_block[k] = blocks;
-        blocks += film_range_blocks(range_start[k + 1] - range_start[k]);
+        blocks += film_range_blocks(range_start[k + 1] - range_start[k], rows_per_block);
     }
     for (int k = num_ranges; k <= kMaxRanges; ++k) {
         R.start[k] = range_start[num_ranges];
         R.first_block[k] = blocks;
     }
+    R.rows_per_block = rows_per_block;
     R.num = num_ranges;
     return R;
 }
 
-// Most phases whose threads fit one workgroup (at most kMaxPhases), and the
-// workgroup size: a multiple of the wave.  Narrow rows take many phases, so
-// that a block of kRowsPerBlock rows still fills a workgroup (rows of 32
-// floats: 16 column pairs x 64 phases of 8 rows each).  With 4 floats per
-// lane the phases' threads stay within 768, so that the backward's fp64
-// phase sums (phases * units * V * 16 bytes) fit 48 KB of LDS.
-constexpr int kMaxPhases = 64;
-FilmLayout film_layout(int64_t units, int V) {
-    const int64_t cap = V >= 4 ? 768 : kMaxThreads;
-    FilmLayout L{static_cast<int>(units), 1};
-    if (units <= cap / 2) L.phases = static_cast<int>(std::min<int64_t>(kMaxPhases, cap / units));
+// Units of a workgroup: all of a row's up to 64 (1 KB of a row with 16-byte
+// units), else an even split of the row into chunks of at most 64, so that no
+// chunk is nearly empty (100 units: 2 chunks of 50, 5 phases each, 250 of 256
+// threads busy).
+FilmLayout film_layout(int64_t width, int V) {
+    const int64_t total = (width + V - 1) / V;
+    FilmLayout L{static_cast<int>(total), static_cast<int>((total + 63) / 64), 0, 0};
+    L.units = static_cast<int>((total + L.chunks - 1) / L.chunks);
+    L.phases = kThreads / L.units;
     return L;
 }
 
-int film_threads(const FilmLayout& L) {
-    const int n = L.units * L.phases;
-    return std::min(kMaxThreads, (n + 63) / 64 * 64);
+// Rows of a workgroup: from `least` to `most` per thread, as many as leave four
+// workgroups to every CU.
+int64_t film_rows_per_block(const FilmLayout& L, int64_t rows, int least, int most) {
+    int per_thread = most;
+    while (per_thread > least && rows * L.chunks < 4 * kCus * per_thread * L.phases) per_thread /= 2;
+    return static_cast<int64_t>(per_thread) * L.phases;
 }
 
-size_t film_lds_bytes(const FilmLayout& L, int V) {
-    return L.phases > 1 ? static_cast<size_t>(L.phases) * L.units * V * 2 * sizeof(double) : 0;
+// 4 floats to a unit, at any alignment; rows narrower than that go one by one.
+int film_vec(int64_t width) { return width >= 4 ? 4 : 1; }
+
+hipError_t film_backward(const float* s, const float* dy, int64_t width, const FilmRanges& R,
+                         const FilmLayout& L, int V, const float* gamma, const float* beta,
+                         const float* add, float* ds, double* partial, hipStream_t st) {
+    const dim3 grid(static_cast<unsigned>(R.first_block[kMaxRanges] * L.chunks));
+    const size_t lds = static_cast<size_t>(L.phases) * L.units * V * 2 * sizeof(double);
+    const auto kernel = V == 4 ? k_film_mish_backward<4> : k_film_mish_backward<1>;
+    hipLaunchKernelGGL(kernel, grid, dim3(kThreads), lds, st, s, dy, width, R, L, gamma, beta, add, ds, partial);
+    return hipGetLastError();
+}
+
+// The split of relm_mp_film_mish_backward_sums: 8 to 64 rows per thread (the
+// blocks' sums are read again, 16 bytes per column and block).
+int64_t film_backward_rows(int64_t width, int64_t rows) {
+    return film_rows_per_block(film_layout(width, film_vec(width)), rows, 8, 64);
 }
 
 }  // namespace
@@ -291,18 +346,14 @@ size_t film_lds_bytes(const FilmLayout& L, int V) {
 hipError_t launch_film_mish(const float* s, int64_t width, const int64_t* range_start,
                             int32_t num_ranges, const float* gamma, const float* beta,
                             const float* add, float* y, hipStream_t st) {
-    const FilmRanges R = film_ranges(range_start, num_ranges);
-    const int64_t blocks = R.first_block[kMaxRanges];
-    if (blocks == 0 || width == 0) return hipSuccess;
-    const int V = film_vec(width, {s, gamma, beta, add, y});
-    const FilmLayout L = film_layout(width / V, V);
-    auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(film_threads(L)), 0, st, s,
-                           width, R, L, gamma, beta, add, y);
-    };
-    if (V == 4) launch(k_film_mish<4>);
-    else if (V == 2) launch(k_film_mish<2>);
-    else launch(k_film_mish<1>);
+    const int64_t rows = range_start[num_ranges];
+    if (rows == 0 || width == 0) return hipSuccess;
+    const int V = film_vec(width);
+    const FilmLayout L = film_layout(width, V);
+    const FilmRanges R = film_ranges(range_start, num_ranges, film_rows_per_block(L, rows, 4, 16));
+    const dim3 grid(static_cast<unsigned>(R.first_block[kMaxRanges] * L.chunks));
+    const auto kernel = V == 4 ? k_film_mish<4> : k_film_mish<1>;
+    hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, st, s, width, R, L, gamma, beta, add, y);
     return hipGetLastError();
 }
 
@@ -310,18 +361,33 @@ hipError_t launch_film_mish_backward(const float* s, const float* dy, int64_t wi
                                      const int64_t* range_start, int32_t num_ranges,
                                      const float* gamma, const float* beta, const float* add,
                                      float* ds, double* partial, hipStream_t st) {
-    const FilmRanges R = film_ranges(range_start, num_ranges);
-    const int64_t blocks = R.first_block[kMaxRanges];
-    if (blocks == 0 || width == 0) return hipSuccess;
-    const int V = film_vec(width, {s, dy, gamma, beta, add, ds, partial});
-    const FilmLayout L = film_layout(width / V, V);
-    auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(blocks)), dim3(film_threads(L)),
-                           film_lds_bytes(L, V), st, s, dy, width, R, L, gamma, beta, add, ds, partial);
-    };
-    if (V == 4) launch(k_film_mish_backward<4>);
-    else if (V == 2) launch(k_film_mish_backward<2>);
-    else launch(k_film_mish_backward<1>);
+    if (range_start[num_ranges] == 0 || width == 0) return hipSuccess;
+    const int V = film_vec(width);
+    const FilmRanges R = film_ranges(range_start, num_ranges, RELM_MP_FILM_ROWS_PER_BLOCK);
+    return film_backward(s, dy, width, R, film_layout(width, V), V, gamma, beta, add, ds, partial, st);
+}
+
+size_t film_sums_workspace(const int64_t* range_start, int32_t num_ranges, int64_t width) {
+    if (range_start[num_ranges] == 0 || width == 0) return 0;
+    const FilmRanges R = film_ranges(range_start, num_ranges, film_backward_rows(width, range_start[num_ranges]));
+    return static_cast<size_t>(R.first_block[kMaxRanges]) * 2 * width * sizeof(double);
+}
+
+hipError_t launch_film_mish_backward_sums(const float* s, const float* dy, int64_t width,
+                                          const int64_t* range_start, int32_t num_ranges,
+                                          const float* gamma, const float* beta, const float* add,
+                                          float* ds, float* sums, double* partial, hipStream_t st) {
+    if (width == 0) return hipSuccess;
+    const int64_t rows = range_start[num_ranges];
+    const int V = film_vec(width);
+    const FilmRanges R = film_ranges(range_start, num_ranges, film_backward_rows(width, rows));
+    if (rows > 0) {
+        const hipError_t e = film_backward(s, dy, width, R, film_layout(width, V), V, gamma, beta, add, ds, partial, st);
+        if (e != hipSuccess) return e;
+    }
+    const int64_t cols = 2 * width;
+    hipLaunchKernelGGL(k_film_fold, dim3(static_cast<unsigned>((cols + kFoldCols - 1) / kFoldCols), num_ranges),
+                       dim3(kThreads), 0, st, partial, cols, R, sums);
     return hipGetLastError();
 }
 

@@ -159,9 +159,9 @@ hipError_t launch_pack_index(const relm_mp_index_part* parts, int num_parts, int
 
 // ---- FiLM step with Mish (film_kernels.hip) ---------------------------------
 constexpr int kFilmMaxRanges = RELM_MP_FILM_MAX_RANGES;
-// Blocks of RELM_MP_FILM_ROWS_PER_BLOCK rows of a range of `rows` rows.
-inline int64_t film_range_blocks(int64_t rows) {
-    return rows <= 0 ? 0 : (rows + RELM_MP_FILM_ROWS_PER_BLOCK - 1) / RELM_MP_FILM_ROWS_PER_BLOCK;
+// Blocks of `per_block` rows of a range of `rows` rows.
+inline int64_t film_range_blocks(int64_t rows, int64_t per_block = RELM_MP_FILM_ROWS_PER_BLOCK) {
+    return rows <= 0 ? 0 : (rows + per_block - 1) / per_block;
 }
 // range_start: num_ranges + 1 ascending host values from 0 to the row count
 // (checked by the caller).
@@ -172,6 +172,13 @@ hipError_t launch_film_mish_backward(const float* s, const float* dy, int64_t wi
                                      const int64_t* range_start, int32_t num_ranges,
                                      const float* gamma, const float* beta, const float* add,
                                      float* ds, double* partial, hipStream_t st);
+// The backward with the blocks' sums added up per range into sums [num_ranges, 2,
+// width]; `partial` holds film_sums_workspace(...) bytes.
+size_t film_sums_workspace(const int64_t* range_start, int32_t num_ranges, int64_t width);
+hipError_t launch_film_mish_backward_sums(const float* s, const float* dy, int64_t width,
+                                          const int64_t* range_start, int32_t num_ranges,
+                                          const float* gamma, const float* beta, const float* add,
+                                          float* ds, float* sums, double* partial, hipStream_t st);
 
 // ---- content comparison (match_kernels.hip) -------------------------------
 constexpr int kMaxMatch = RELM_MP_MAX_MATCH;

@@ -1838,30 +1838,17 @@ std::tuple<Tensor, Tensor, Tensor> film_mish_backward(const Tensor& grad, const 
     const Tensor g = contiguous(grad);
     const int32_t k = static_cast<int32_t>(a.starts.size() - 1);
     const int64_t width = a.s.size(1);
-    const int64_t blocks = relm_mp_film_mish_blocks(a.starts.data(), k);
-    TORCH_CHECK(blocks >= 0, "film_mish_backward: bad row ranges.");
+    TORCH_CHECK(relm_mp_film_mish_blocks(a.starts.data(), k) >= 0, "film_mish_backward: bad row ranges.");
     Tensor ds = at::empty_like(a.s);
-    Tensor partial = at::empty({std::max<int64_t>(blocks, 1), 2, width}, a.s.options().dtype(at::kDouble));
-    raise_if(relm_mp_film_mish_backward(fptr(a.s), g.data_ptr<float>(), a.s.size(0), width,
-                                        a.starts.data(), k, fptr(a.gamma), fptr(a.beta), fptr(a.add),
-                                        ds.data_ptr<float>(), partial.data_ptr<double>(), blocks,
-                                        current_stream(a.s)));
-    // per range, the sums of its blocks (consecutive, RELM_MP_FILM_ROWS_PER_BLOCK
-    // rows each) in fp64, rounded to fp32 once
-    if (k == 1 && blocks > 0) {
-        const Tensor sum = partial.sum(0).to(at::kFloat);  // [2, width]
-        return {ds, sum.narrow(0, 0, 1), sum.narrow(0, 1, 1)};
-    }
-    Tensor sums = at::zeros({k, 2, width}, partial.options());
-    int64_t b0 = 0;
-    for (int32_t r = 0; r < k; ++r) {
-        const int64_t rows = a.starts[r + 1] - a.starts[r];
-        const int64_t nb = rows <= 0 ? 0 : (rows + RELM_MP_FILM_ROWS_PER_BLOCK - 1) / RELM_MP_FILM_ROWS_PER_BLOCK;
-        if (nb > 0) sums[r].copy_(partial.narrow(0, b0, nb).sum(0));
-        b0 += nb;
-    }
-    const Tensor sums32 = sums.to(at::kFloat);
-    return {ds, sums32.select(1, 0), sums32.select(1, 1)};
+    // per range the column sums, added in fp64 and rounded to fp32 once
+    Tensor sums = at::empty({k, 2, width}, a.s.options());
+    const size_t bytes = relm_mp_film_mish_backward_sums_workspace_size(a.starts.data(), k, width);
+    Tensor partial = at::empty({static_cast<int64_t>(bytes)}, a.s.options().dtype(at::kByte));
+    raise_if(relm_mp_film_mish_backward_sums(fptr(a.s), g.data_ptr<float>(), a.s.size(0), width,
+                                             a.starts.data(), k, fptr(a.gamma), fptr(a.beta), fptr(a.add),
+                                             ds.data_ptr<float>(), sums.data_ptr<float>(),
+                                             partial.data_ptr(), bytes, current_stream(a.s)));
+    return {ds, sums.select(1, 0), sums.select(1, 1)};
 }
 
 // ---- a @ b^T for the models' narrow Linears (no counterpart in the reference) ----

@@ -131,6 +131,36 @@ def test_film_mish_bitwise_against_torch_over_float_ranges(lo_bits: int, hi_bits
     assert bool(same.all()), u[~same][:8].tolist()
 
 
+@pytest.mark.parametrize("width,starts", [
+    (1, [0, 1]),                       # rows narrower than one unit
+    (3, [0, 5, 5, 1300]),
+    (5, [0, 70, 4099]),                # the last unit shares columns with the one before
+    (64, [0, 0, 16, 17, 1041]),        # empty and one-row ranges
+    (257, [0, 129, 20000]),            # two column chunks, the second shorter
+    (400, [0, 33]),
+])
+def test_film_mish_backward_sums(width, starts) -> None:
+    """The column sums added up on the device: the block sums of the 512-row
+    split added in fp64 (fp32 terms in another fp64 order: equal but for a
+    rounding on the edge of two floats), exactly zero for an empty range, and
+    the same input gradient."""
+
+    from relmo_amd import capi
+
+    g = torch.Generator(device=DEV).manual_seed(width)
+    k, rows = len(starts) - 1, starts[-1]
+    s, dy = (torch.randn(rows, width, device=DEV, generator=g) for _ in range(2))
+    gamma, beta, add = (torch.randn(k, width, device=DEV, generator=g) for _ in range(3))
+    ds, sums = capi.film_mish_backward_sums(dy, s, starts, gamma, beta, add)
+    ds_blocks, partial = capi.film_mish_backward(dy, s, starts, gamma, beta, add)
+    assert torch.equal(ds, ds_blocks)
+    b0 = 0
+    for r in range(k):
+        nb = -(-(starts[r + 1] - starts[r]) // 512)
+        torch.testing.assert_close(sums[r], partial[b0:b0 + nb].sum(0).float(), rtol=1.2e-7, atol=0)
+        b0 += nb
+
+
 def test_film_mish_extremes_and_errors() -> None:
     """Large and very negative pre-activations (Mish is u and 0 there), and
     ranges that do not cover the rows."""
