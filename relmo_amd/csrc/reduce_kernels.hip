@@ -1,9 +1,9 @@
 // Row kernels of the relational message-passing ops.
 //
 // Every output row is owned by exactly one "row group" of G lanes (G = 4..64,
-// a divisor of the wave), each lane moving V contiguous elements (float4 /
-// double2 when the rows allow it); rows wider than G*V are split over
-// blockIdx.y slices.  No atomics anywhere: the messages of a key are visited
+// a divisor of the wave), each lane moving V contiguous elements (16 bytes;
+// one element where a row is narrower than that) at any alignment; rows wider
+// than G*V are split over blockIdx.y slices.  No atomics anywhere: the messages of a key are visited
 // in the stable (edge) order of the plan, so every result is deterministic.
 //
 // CSR plans are reduced in two parts:
@@ -47,6 +47,18 @@ constexpr int64_t kMaxBlocksX = 1 << 22;  // keeps blocks * 1024 threads below 2
 // Largest pair of arrays read into the memory-side cache (256 MB on MI355X)
 // ahead of a write-dominated kernel.
 constexpr size_t kPrefetchMaxBytes = size_t(256) << 20;
+
+// First column of lane `gl` of a row group, or D or more for a lane past the
+// row.  Where V does not divide D the row's last lane is moved back to end with
+// the row; the columns it shares with the lane before are computed twice, with
+// equal results (each column's values and order do not depend on the lane).
+// Rows of 33 floats so take 9 lanes of a group of 16 instead of 33 lanes of 64.
+template <int V, int G>
+__device__ __forceinline__ uint32_t lane_column(int gl, int64_t D) {
+    const uint32_t c = blockIdx.y * (G * V) + static_cast<uint32_t>(gl) * V;
+    const uint32_t d = static_cast<uint32_t>(D);
+    return c < d ? min(c, d - V) : c;
+}
 
 template <int G>
 constexpr int batch_rows() {
@@ -165,9 +177,8 @@ struct SumOp {
     using Partial = SumPartial<T, V>;
     const T* __restrict__ table;
     int64_t D;
-    int64_t col;
-    bool colok;
-    int64_t lcol;  // column the lane loads: col, or 0 past the row (value unused)
+    uint32_t col;  // first column of the lane; 0 past the row (the values are not used)
+    bool colok;   // the lane has columns
     Pack<T, V> x[U];
     Pack<T, V> acc;
     Rows rows;  // layout of the table rows
@@ -188,7 +199,7 @@ struct SumOp {
     // accumulated, lanes past the row never stored.
     __device__ __forceinline__ void load(const int32_t (&idx)[U], int) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) x[u] = pack_load<T, V>(table + rows(idx[u], D) + lcol);
+        for (int u = 0; u < U; ++u) x[u] = pack_load<T, V>(table + rows(idx[u], D) + col);
     }
     // Rows u >= cnt (or !valid) leave the accumulator as it is: selects, not
     // branches, so the loads stay unconditional.
@@ -247,9 +258,8 @@ struct LseOp {
     using Partial = LsePartial<T, V>;
     const T* __restrict__ table;
     int64_t D;
-    int64_t col;
+    uint32_t col;
     bool colok;
-    int64_t lcol;  // as SumOp::lcol
     Pack<T, V> x[U];
     Pack<T, V> m, s;
 
@@ -276,7 +286,7 @@ struct LseOp {
     // as SumOp::load
     __device__ __forceinline__ void load(const int32_t (&idx)[U], int) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) x[u] = pack_load<T, V>(table + row_offset(idx[u], D) + lcol);
+        for (int u = 0; u < U; ++u) x[u] = pack_load<T, V>(table + row_offset(idx[u], D) + col);
     }
     // Batch maximum, then the rescaled sum; rows u >= cnt are masked by
     // selects (no branch, so the loads stay unconditional).  While the maximum
@@ -348,16 +358,15 @@ struct LseBwdOp {
     const T* __restrict__ out;
     const T* __restrict__ rel;
     int64_t D;
-    int64_t col;
+    uint32_t col;
     bool colok;
-    int64_t lcol;  // as SumOp::lcol
     Pack<T, V> g[U], o[U];
     Pack<T, V> xr, acc;
 
     // key is a valid rel row (hub chunks outside the plan pass row 0)
     __device__ __forceinline__ void begin(int64_t key, bool) {
         acc = pack_fill<T, V>(T(0));
-        xr = pack_load<T, V>(rel + key * D + lcol);
+        xr = pack_load<T, V>(rel + key * D + col);
     }
     __device__ __forceinline__ void restart(bool head, int64_t key) {
         if (head) begin(key, true);
@@ -366,7 +375,7 @@ struct LseBwdOp {
     __device__ __forceinline__ void load(const int32_t (&idx)[U], int) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const uint64_t off = row_offset(idx[u], D) + lcol;
+            const uint64_t off = row_offset(idx[u], D) + col;
             g[u] = pack_load<T, V>(grad_out + off);
             o[u] = pack_load<T, V>(out + off);
         }
@@ -390,29 +399,30 @@ struct LseBwdOp {
 
 // ---- epilogues: applied to each key's result as it is stored ----------------
 
-// Stores the result as is.
 // Minimum waves per SIMD asked of the compiler for the walker and the hub
 // chunks (HIP's second launch bound), which caps their VGPRs: the fp32 sum and
 // logsumexp over dense rows fit 96 VGPRs in the walker (5 waves instead of 4 at
-// 116) and 80 in the hub chunks (6 instead of 5 at 93) without spilling; the
+// 116), the sum of rows of more than 32 floats 80 (6 waves; narrower ones would
+// spill), and 80 in the hub chunks (6 instead of 5 at 93) without spilling; the
 // other ops (fp64, grouped rows, the logsumexp backward) would spill, and keep
 // the compiler's choice.
-template <class Op>
+template <class Op, int G>
 struct WaveFloor {
     static constexpr int walk = 1;
     static constexpr int hub = 1;
 };
-template <int V, int U>
-struct WaveFloor<SumOp<float, V, U, DenseRows>> {
-    static constexpr int walk = 5;
+template <int V, int U, int G>
+struct WaveFloor<SumOp<float, V, U, DenseRows>, G> {
+    static constexpr int walk = G >= 16 ? 6 : 5;
     static constexpr int hub = 6;
 };
-template <int V, int U>
-struct WaveFloor<LseOp<float, V, U>> {
+template <int V, int U, int G>
+struct WaveFloor<LseOp<float, V, U>, G> {
     static constexpr int walk = 5;
     static constexpr int hub = 6;
 };
 
+// Stores the result as is.
 struct NoEpilogue {
     template <typename T, int V>
     __device__ __forceinline__ Pack<T, V> operator()(int64_t, const Pack<T, V>& v, int64_t,
@@ -487,7 +497,7 @@ __global__ __launch_bounds__(kThreads) void k_fill(T* __restrict__ p, int64_t n,
 // whose label differs from the next one stores its key's result - no
 // per-key loop, so the row groups of a wave stay in step.
 template <typename T, int V, int G, class Op, class Epi>
-__global__ __launch_bounds__(kThreads, WaveFloor<Op>::walk) void k_walk_items(
+__global__ __launch_bounds__(kThreads, (WaveFloor<Op, G>::walk)) void k_walk_items(
     const int32_t* __restrict__ short_off, const int32_t* __restrict__ short_gather_in,
     const int32_t* __restrict__ gather_sorted, const int32_t* __restrict__ item_first,
     const int32_t* __restrict__ item_short, const relm_mp_plan_counts* __restrict__ pc,
@@ -511,9 +521,9 @@ __global__ __launch_bounds__(kThreads, WaveFloor<Op>::walk) void k_walk_items(
     __shared__ uint32_t s_scan[kThreads / kWave];
     const int gl = static_cast<int>(threadIdx.x) & (G - 1);
     const int grp = static_cast<int>(threadIdx.x) / G;
-    op.col = static_cast<int64_t>(blockIdx.y) * (G * V) + static_cast<int64_t>(gl) * V;
-    op.colok = op.col < op.D;
-    op.lcol = op.colok ? op.col : 0;
+    const uint32_t lane_col = lane_column<V, G>(gl, op.D);
+    op.colok = lane_col < op.D;
+    op.col = op.colok ? lane_col : 0;
     const int64_t D = op.D;
     const int64_t num_items = pc->num_items;
     const int64_t num_short = pc->num_short;
@@ -700,7 +710,7 @@ __device__ __forceinline__ int hub_slot(int p) { return p + (p >> 5); }
 // LDS with coalesced loads, row group g folds slice g of the chunk, the
 // slices are folded in order by group 0; a single-chunk hub is finished here.
 template <typename T, int V, int G, class Op, class Epi>
-__global__ __launch_bounds__(kThreads, WaveFloor<Op>::hub) void k_hub_chunks(
+__global__ __launch_bounds__(kThreads, (WaveFloor<Op, G>::hub)) void k_hub_chunks(
     const int32_t* __restrict__ offsets, const int32_t* __restrict__ gs, int64_t num_edges,
     const int32_t* __restrict__ hub_key, const int32_t* __restrict__ hub_chunk_base,
     const int32_t* __restrict__ chunk_hub, const relm_mp_plan_counts* __restrict__ pc,
@@ -713,9 +723,9 @@ __global__ __launch_bounds__(kThreads, WaveFloor<Op>::hub) void k_hub_chunks(
     __shared__ int32_t s_gs[kChunkSize + kChunkSize / 32];
     const int gl = static_cast<int>(threadIdx.x) & (G - 1);
     const int grp = static_cast<int>(threadIdx.x) / G;
-    op.col = static_cast<int64_t>(blockIdx.y) * (G * V) + static_cast<int64_t>(gl) * V;
-    op.colok = op.col < op.D;
-    op.lcol = op.colok ? op.col : 0;
+    const uint32_t lane_col = lane_column<V, G>(gl, op.D);
+    op.colok = lane_col < op.D;
+    op.col = op.colok ? lane_col : 0;
     const int64_t D = op.D;
     const int64_t num_hubs = pc->num_hubs;
     const int64_t num_chunks = pc->num_chunks;
@@ -805,7 +815,7 @@ __global__ __launch_bounds__(kThreads) void k_hub_combine(
     __shared__ Partial red[kThreads / kWave * G];
     const int gl = static_cast<int>(threadIdx.x) & (G - 1);
     const int grp = static_cast<int>(threadIdx.x) / G;
-    const int64_t col = static_cast<int64_t>(blockIdx.y) * (G * V) + static_cast<int64_t>(gl) * V;
+    const uint32_t col = lane_column<V, G>(gl, D);
     const bool colok = col < D;
     const int64_t num_hubs = pc->num_hubs;
     const int64_t num_multi_hubs = pc->num_multi_hubs;
@@ -902,18 +912,12 @@ struct InvRow {
     bool ok;       // the row has an edge whose gathered index is in [0, num_gather)
 };
 
+// Fills in g and ok of rows whose key and live are set.
 template <int RU, class Src>
-__device__ __forceinline__ void inverse_rows(InvRow (&r)[RU], int64_t key0, int64_t stride,
-                                             const int32_t* __restrict__ inv, int64_t num_keys,
-                                             int64_t num_edges, const Src& gathers,
-                                             int64_t num_gather) {
+__device__ __forceinline__ void inverse_gather(InvRow (&r)[RU], const int32_t* __restrict__ inv,
+                                               int64_t num_edges, const Src& gathers,
+                                               int64_t num_gather) {
     int64_t e[RU];
-#pragma unroll
-    for (int j = 0; j < RU; ++j) {
-        const int64_t key = key0 + j * stride;
-        r[j].live = key < num_keys;
-        r[j].key = r[j].live ? key : 0;
-    }
     if (inv != nullptr) {
 #pragma unroll
         for (int j = 0; j < RU; ++j) {
@@ -939,6 +943,20 @@ __device__ __forceinline__ void inverse_rows(InvRow (&r)[RU], int64_t key0, int6
     }
 }
 
+template <int RU, class Src>
+__device__ __forceinline__ void inverse_rows(InvRow (&r)[RU], int64_t key0, int64_t stride,
+                                             const int32_t* __restrict__ inv, int64_t num_keys,
+                                             int64_t num_edges, const Src& gathers,
+                                             int64_t num_gather) {
+#pragma unroll
+    for (int j = 0; j < RU; ++j) {
+        const int64_t key = key0 + j * stride;
+        r[j].live = key < num_keys;
+        r[j].key = r[j].live ? key : 0;
+    }
+    inverse_gather<RU>(r, inv, num_edges, gathers, num_gather);
+}
+
 template <typename T, int V, int G, class Rows, class Src>
 __global__ __launch_bounds__(kThreads) void k_gather_inv(const int32_t* __restrict__ inv_in,
                                                          const relm_mp_plan_counts* __restrict__ pc,
@@ -953,7 +971,7 @@ __global__ __launch_bounds__(kThreads) void k_gather_inv(const int32_t* __restri
     // an inverse map built without atomics is only used when no row repeats
     if (skip_on_collision && pc->collisions != 0) return;
     const int gl = static_cast<int>(threadIdx.x) & (G - 1);
-    const int64_t col = static_cast<int64_t>(blockIdx.y) * (G * V) + static_cast<int64_t>(gl) * V;
+    const uint32_t col = lane_column<V, G>(gl, D);
     if (col >= D) return;
     const int32_t* inv = inverse_map(inv_in, pc);
     const int64_t chunk = static_cast<int64_t>(R) * RU;
@@ -976,6 +994,158 @@ __global__ __launch_bounds__(kThreads) void k_gather_inv(const int32_t* __restri
         for (int j = 0; j < RU; ++j) {
             if (!r[j].ok) v[j] = pack_fill<T, V>(T(0));
             if (r[j].live) pack_store_stream<T, V>(out + out_rows(r[j].key, D) + col, v[j]);
+        }
+    }
+}
+
+// Rows whose size is no multiple of 16 bytes: the output as one flat array in
+// aligned pieces of 16 bytes, each the end of one row and the start of the next
+// where it lies across their seam.  Every lane stores a whole piece, so the
+// stores fill whole lines; a row to a row group stores pieces of lines that its
+// neighbours complete later: the sum backward of 3 M messages of 33 floats takes
+// 180 us in pieces, 278 us by rows in 4-byte lanes and 309 in 16-byte ones.  A
+// thread keeps kFlatPieces pieces in flight.
+constexpr int kFlatPieces = 4;
+constexpr int64_t kFlatMaxColumns = 4096;  // n / D below by one 32-bit multiply: n < D + 4096, both below 2^16
+
+template <int V>
+struct FlatPiece {
+    int64_t at;    // first element in the output
+    int64_t left;  // elements of the output from there on, <= 0 past its end
+    int col;       // column of the first element
+    int over;      // elements that belong to the next row
+};
+
+// Pieces of this thread in the chunk of kThreads * kFlatPieces * V elements at
+// f0, and their rows: r[2 j] the first row of piece j, r[2 j + 1] the second
+// (the first again where the piece lies in one row).
+template <int V>
+__device__ __forceinline__ void flat_pieces(FlatPiece<V> (&p)[kFlatPieces], InvRow (&r)[2 * kFlatPieces],
+                                            int64_t f0, int64_t num_keys, int32_t D, uint32_t magic) {
+    const int64_t row0 = f0 / D;
+    const uint32_t rem = static_cast<uint32_t>(f0 - row0 * D);
+    const int64_t total = num_keys * D;
+#pragma unroll
+    for (int j = 0; j < kFlatPieces; ++j) {
+        const uint32_t o = static_cast<uint32_t>(j * kThreads + static_cast<int>(threadIdx.x)) * V;
+        const uint32_t q = __umulhi(rem + o, magic);
+        p[j].at = f0 + o;
+        p[j].left = total - p[j].at;
+        p[j].col = static_cast<int>(rem + o - q * static_cast<uint32_t>(D));
+        p[j].over = max(p[j].col + V - D, 0);
+        const int64_t row = row0 + q;
+        const bool two = p[j].over > 0 && row + 1 < num_keys;
+        r[2 * j].live = r[2 * j + 1].live = row < num_keys;
+        r[2 * j].key = row < num_keys ? row : 0;
+        r[2 * j + 1].key = r[2 * j].key + (two ? 1 : 0);
+    }
+}
+
+// The V elements from column `col` of table row a and on into row b: row a's
+// last V elements, and row b's first ones moved in behind them.
+template <typename T, int V>
+__device__ __forceinline__ Pack<T, V> flat_load(const T* __restrict__ table, int64_t D, const InvRow& a,
+                                                const InvRow& b, int col, int over) {
+    const Pack<T, V> x = pack_load<T, V>(table + row_offset(a.g, D) + (col - over));
+    Pack<T, V> y = x;
+    if (over > 0) y = pack_load<T, V>(table + row_offset(b.g, D));
+    T w[2 * V];
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+        w[i] = a.ok ? x.v[i] : T(0);
+        w[V + i] = b.ok ? y.v[i] : T(0);
+    }
+#pragma unroll
+    for (int s = 1; s < V; s *= 2) {
+        const bool shift = (over & s) != 0;
+#pragma unroll
+        for (int i = 0; i + s < 2 * V; ++i) w[i] = shift ? w[i + s] : w[i];
+    }
+    Pack<T, V> v;
+#pragma unroll
+    for (int i = 0; i < V; ++i) v.v[i] = w[i];
+    return v;
+}
+
+template <typename T, int V>
+__device__ __forceinline__ void flat_store(T* __restrict__ out, const FlatPiece<V>& p, const Pack<T, V>& v) {
+    if (p.left >= V) {
+        pack_store_stream<T, V>(out + p.at, v);
+    } else {
+#pragma unroll
+        for (int i = 0; i < V; ++i)
+            if (i < p.left) out[p.at + i] = v.v[i];
+    }
+}
+
+// k_gather_inv by flat pieces (V < D <= kFlatMaxColumns).
+template <typename T, class Src>
+__global__ __launch_bounds__(kThreads) void k_gather_flat(const int32_t* __restrict__ inv_in,
+                                                          const relm_mp_plan_counts* __restrict__ pc,
+                                                          int64_t num_edges, Src gathers, int64_t num_gather,
+                                                          const T* __restrict__ table, int64_t num_keys,
+                                                          int32_t D, uint32_t magic, T* __restrict__ out,
+                                                          bool skip_on_collision) {
+    constexpr int V = 16 / static_cast<int>(sizeof(T));
+    constexpr int64_t kChunk = static_cast<int64_t>(kThreads) * kFlatPieces * V;
+    if (skip_on_collision && pc->collisions != 0) return;
+    const int32_t* inv = inverse_map(inv_in, pc);
+    for (int64_t f0 = blockIdx.x * kChunk; f0 < num_keys * D; f0 += gridDim.x * kChunk) {
+        FlatPiece<V> p[kFlatPieces];
+        InvRow r[2 * kFlatPieces];
+        flat_pieces<V>(p, r, f0, num_keys, D, magic);
+        inverse_gather(r, inv, num_edges, gathers, num_gather);
+        Pack<T, V> v[kFlatPieces];
+#pragma unroll
+        for (int j = 0; j < kFlatPieces; ++j)
+            v[j] = flat_load<T, V>(table, D, r[2 * j], r[2 * j + 1], p[j].col, p[j].over);
+#pragma unroll
+        for (int j = 0; j < kFlatPieces; ++j) flat_store<T, V>(out, p[j], v[j]);
+    }
+}
+
+// k_lse_bwd_inv by flat pieces.
+template <typename T, class Src>
+__global__ __launch_bounds__(kThreads) void k_lse_bwd_flat(const int32_t* __restrict__ inv_in,
+                                                           const relm_mp_plan_counts* __restrict__ pc,
+                                                           int64_t num_edges, Src gathers, int64_t num_gather,
+                                                           const T* __restrict__ grad_out,
+                                                           const T* __restrict__ out, const T* __restrict__ rel,
+                                                           int64_t num_keys, int32_t D, uint32_t magic,
+                                                           T* __restrict__ grad_rel, bool skip_on_collision) {
+    constexpr int V = 16 / static_cast<int>(sizeof(T));
+    constexpr int64_t kChunk = static_cast<int64_t>(kThreads) * kFlatPieces * V;
+    if (skip_on_collision && pc->collisions != 0) return;
+    const int32_t* inv = inverse_map(inv_in, pc);
+    for (int64_t f0 = blockIdx.x * kChunk; f0 < num_keys * D; f0 += gridDim.x * kChunk) {
+        FlatPiece<V> p[kFlatPieces];
+        InvRow r[2 * kFlatPieces];
+        flat_pieces<V>(p, r, f0, num_keys, D, magic);
+        inverse_gather(r, inv, num_edges, gathers, num_gather);
+        Pack<T, V> x[kFlatPieces], g[kFlatPieces], o[kFlatPieces];
+#pragma unroll
+        for (int j = 0; j < kFlatPieces; ++j) {
+            // the last piece may end behind the rows: read one that does not
+            const int64_t back = p[j].left >= V ? 0 : V - p[j].left;
+            x[j] = pack_load_stream<T, V>(rel + (p[j].left > 0 ? p[j].at - back : 0));
+            if (p[j].left > 0 && back > 0) {
+#pragma unroll
+                for (int i = 0; i < V; ++i) x[j].v[i] = rel[i < p[j].left ? p[j].at + i : p[j].at];
+            }
+            g[j] = flat_load<T, V>(grad_out, D, r[2 * j], r[2 * j + 1], p[j].col, p[j].over);
+            o[j] = flat_load<T, V>(out, D, r[2 * j], r[2 * j + 1], p[j].col, p[j].over);
+        }
+#pragma unroll
+        for (int j = 0; j < kFlatPieces; ++j) {
+            Pack<T, V> res;
+#pragma unroll
+            for (int i = 0; i < V; ++i) {
+                const bool ok = i < V - p[j].over ? r[2 * j].ok : r[2 * j + 1].ok;
+                const T w = fast_exp<T>(x[j].v[i] - o[j].v[i]);
+                const T c = g[j].v[i] * w;
+                res.v[i] = ok ? T(0) + c : T(0);
+            }
+            flat_store<T, V>(grad_rel, p[j], res);
         }
     }
 }
@@ -1011,7 +1181,7 @@ __global__ __launch_bounds__(kThreads) void k_rows_scale(
     constexpr int R = kThreads / G;
     constexpr int RU = gather_rows_in_flight<T, V>();
     const int gl = static_cast<int>(threadIdx.x) & (G - 1);
-    const int64_t col = static_cast<int64_t>(blockIdx.y) * (G * V) + static_cast<int64_t>(gl) * V;
+    const uint32_t col = lane_column<V, G>(gl, D);
     if (col >= D) return;
     const int64_t chunk = static_cast<int64_t>(R) * RU;
     for (int64_t r0 = static_cast<int64_t>(blockIdx.x) * chunk + threadIdx.x / G; r0 < rows;
@@ -1063,7 +1233,7 @@ __global__ __launch_bounds__(kThreads) void k_gather_last_csr(const int32_t* __r
                                                               T* __restrict__ out, Rows out_rows) {
     constexpr int R = kThreads / G;
     const int gl = static_cast<int>(threadIdx.x) & (G - 1);
-    const int64_t col = static_cast<int64_t>(blockIdx.y) * (G * V) + static_cast<int64_t>(gl) * V;
+    const uint32_t col = lane_column<V, G>(gl, D);
     if (col >= D) return;
     for (int64_t key = static_cast<int64_t>(blockIdx.x) * R + threadIdx.x / G; key < num_keys;
          key += static_cast<int64_t>(gridDim.x) * R) {
@@ -1089,7 +1259,7 @@ __global__ __launch_bounds__(kThreads) void k_lse_bwd_inv(
     // an inverse map built without atomics is only used when no row repeats
     if (skip_on_collision && pc->collisions != 0) return;
     const int gl = static_cast<int>(threadIdx.x) & (G - 1);
-    const int64_t col = static_cast<int64_t>(blockIdx.y) * (G * V) + static_cast<int64_t>(gl) * V;
+    const uint32_t col = lane_column<V, G>(gl, D);
     if (col >= D) return;
     const int32_t* inv = inverse_map(inv_in, pc);
     const int64_t chunk = static_cast<int64_t>(R) * RU;
@@ -1176,7 +1346,7 @@ __global__ __launch_bounds__(kThreads) void k_gather_edges(const relm_mp_plan_co
     constexpr int RU = gather_rows_in_flight<T, V>();
     if (pc->collisions != 0) return;  // not a permutation: the caller takes another path
     const int gl = static_cast<int>(threadIdx.x) & (G - 1);
-    const int64_t col = static_cast<int64_t>(blockIdx.y) * (G * V) + static_cast<int64_t>(gl) * V;
+    const uint32_t col = lane_column<V, G>(gl, D);
     if (col >= D) return;
     const int64_t chunk = static_cast<int64_t>(R) * RU;
     const int64_t grp = threadIdx.x / G;
@@ -1201,24 +1371,19 @@ struct Geometry {
     int64_t slices;
 };
 
-// Dense rows: the widest of kVecMax, kVecMax / 2 and 1 elements per lane that
-// divides D and keeps every row start aligned (rows of an even number of
-// floats that is not a multiple of 4 still move 8 bytes per lane).
+// 16 bytes per lane whatever the alignment (lane_column), one element where a
+// row has fewer.  Narrower lanes where the rows or the base are not aligned cost
+// more than the straddled lines do: 2 M argument slots of 128 floats at an
+// 8-byte aligned column 575 us in 8-byte lanes, 503 in 16-byte ones; the hub
+// chunks of 3 M messages of 33 floats 120 us in 4-byte lanes, 106 in 16-byte ones.
 template <typename T>
-Geometry choose_geometry(int64_t D, std::initializer_list<const void*> ptrs) {
+Geometry choose_geometry(int64_t D) {
     constexpr int kVecMax = 16 / static_cast<int>(sizeof(T));
-    int V = kVecMax;
-    for (; V > 1; V /= 2) {
-        bool ok = D % V == 0;
-        for (const void* p : ptrs)
-            ok = ok && (p == nullptr || reinterpret_cast<uintptr_t>(p) % (sizeof(T) * V) == 0);
-        if (ok) break;
-    }
+    const int V = D >= kVecMax ? kVecMax : 1;
     const int64_t vcols = (D + V - 1) / V;
     int G = 4;
     while (G < vcols && G < 64) G *= 2;
-    const int64_t slices = (vcols + G - 1) / G;
-    return {V, G, slices};
+    return {V, G, (vcols + G - 1) / G};
 }
 
 template <typename T, typename F>
@@ -1236,49 +1401,6 @@ int with_geometry(const Geometry& geo, F&& f) {
     };
     constexpr int kVecMax = 16 / static_cast<int>(sizeof(T));
     if (geo.V == kVecMax) return by_g(std::integral_constant<int, kVecMax>{});
-    if constexpr (kVecMax > 2) {
-        if (geo.V == kVecMax / 2) return by_g(std::integral_constant<int, kVecMax / 2>{});
-    }
-    return by_g(std::integral_constant<int, 1>{});
-}
-
-// Grouped row layouts (argument slots of a wider matrix): the widest of
-// kVecMax, kVecMax / 2 and 1 elements per lane that keeps every row start
-// aligned - lines of an odd number of 8-byte pairs still move 8 bytes per lane.
-template <typename T>
-Geometry choose_grouped_geometry(int64_t D, int64_t stride, std::initializer_list<const void*> ptrs) {
-    constexpr int kVecMax = 16 / static_cast<int>(sizeof(T));
-    int V = kVecMax;
-    for (; V > 1; V /= 2) {
-        bool ok = D % V == 0 && stride % V == 0;
-        for (const void* p : ptrs)
-            ok = ok && (p == nullptr || reinterpret_cast<uintptr_t>(p) % (sizeof(T) * V) == 0);
-        if (ok) break;
-    }
-    const int64_t vcols = (D + V - 1) / V;
-    int G = 4;
-    while (G < vcols && G < 64) G *= 2;
-    return {V, G, (vcols + G - 1) / G};
-}
-
-template <typename T, typename F>
-int with_grouped_geometry(const Geometry& geo, F&& f) {
-    constexpr int kVecMax = 16 / static_cast<int>(sizeof(T));
-    auto by_g = [&](auto vt) -> int {
-        switch (geo.G) {
-            case 4: return f(vt, std::integral_constant<int, 4>{});
-            case 8: return f(vt, std::integral_constant<int, 8>{});
-            case 16: return f(vt, std::integral_constant<int, 16>{});
-            case 32: return f(vt, std::integral_constant<int, 32>{});
-            case 64: return f(vt, std::integral_constant<int, 64>{});
-            default: break;
-        }
-        return set_error(RELM_MP_ERR_INVALID_ARGUMENT, "relm_mp: unsupported row geometry");
-    };
-    if (geo.V == kVecMax) return by_g(std::integral_constant<int, kVecMax>{});
-    if constexpr (kVecMax > 2) {
-        if (geo.V == kVecMax / 2) return by_g(std::integral_constant<int, kVecMax / 2>{});
-    }
     return by_g(std::integral_constant<int, 1>{});
 }
 
@@ -1289,6 +1411,22 @@ dim3 row_grid(int64_t rows, int G, int64_t slices, int rows_per_group = 1) {
     if (bx > kMaxBlocksX) bx = kMaxBlocksX;
     return dim3(static_cast<unsigned>(bx), static_cast<unsigned>(slices));
 }
+
+// Whether rows of D elements go through the flat kernels.
+template <typename T>
+bool flat_rows(int64_t D, int64_t num_edges, int64_t num_gather) {
+    constexpr int V = 16 / static_cast<int>(sizeof(T));
+    return D > V && D % V != 0 && D <= kFlatMaxColumns && num_edges > 0 && num_gather > 0;
+}
+
+template <typename T>
+dim3 flat_grid(int64_t rows, int64_t D) {
+    constexpr int64_t kChunk = static_cast<int64_t>(kThreads) * kFlatPieces * (16 / sizeof(T));
+    return dim3(static_cast<unsigned>(std::min<int64_t>((rows * D + kChunk - 1) / kChunk, kMaxBlocksX)));
+}
+
+// ceil(2^32 / D): n / D = high word of n * magic for n, D < 2^16.
+uint32_t flat_magic(int64_t D) { return static_cast<uint32_t>(((uint64_t(1) << 32) + D - 1) / D); }
 
 // Workgroups of `kernel` (kThreads each) resident on the current device at
 // once; persistent launches size their grids with it.
@@ -1401,12 +1539,22 @@ int gather_last_t(const relm_mp_plan& plan, const int64_t* gathers, const void* 
         return hip_error(hipGetLastError(), "relm_mp gather kernel");
     };
     if (group > 0) {
-        const Geometry geo = choose_grouped_geometry<T>(emb, group_stride, {table, out});
+        const Geometry geo = choose_geometry<T>(emb);
         const GroupedRows rows{static_cast<uint32_t>(group), static_cast<uint64_t>(group_stride)};
-        return with_grouped_geometry<T>(
+        return with_geometry<T>(
             geo, [&](auto vt, auto gt) -> int { return launch(vt, gt, geo, rows); });
     }
-    const Geometry geo = choose_geometry<T>(emb, {table, out});
+    if (plan.kind == RELM_MP_PLAN_INVERSE && flat_rows<T>(emb, plan.num_edges, plan.num_gather)) {
+        const auto flat = [&](auto src) {
+            hipLaunchKernelGGL((k_gather_flat<T, decltype(src)>), flat_grid<T>(plan.num_keys, emb), dim3(kThreads), 0,
+                               s, plan.inv, plan.counts, plan.num_edges, src, plan.num_gather, table,
+                               plan.num_keys, static_cast<int32_t>(emb), flat_magic(emb), out, skip_on_collision);
+        };
+        if (snap != nullptr) flat(GathersSnap{snap->snap_keys, snap->snap_key_plain});
+        else flat(GathersI64{gathers});
+        return hip_error(hipGetLastError(), "relm_mp gather kernel");
+    }
+    const Geometry geo = choose_geometry<T>(emb);
     return with_geometry<T>(geo,
                             [&](auto vt, auto gt) -> int { return launch(vt, gt, geo, DenseRows{}); });
 }
@@ -1419,8 +1567,8 @@ int segment_sum_grouped_t(const relm_mp_plan& plan, const void* table_v, int64_t
     const T* table = static_cast<const T*>(table_v);
     T* out = static_cast<T*>(out_v);
     T* partial = static_cast<T*>(scratch);
-    const Geometry geo = choose_grouped_geometry<T>(emb, group_stride, {table, out, partial});
-    return with_grouped_geometry<T>(geo, [&](auto vt, auto gt) -> int {
+    const Geometry geo = choose_geometry<T>(emb);
+    return with_geometry<T>(geo, [&](auto vt, auto gt) -> int {
         constexpr int V = decltype(vt)::value;
         constexpr int G = decltype(gt)::value;
         constexpr int U = batch_rows<G>();
@@ -1438,7 +1586,7 @@ int segment_reduce_t(const relm_mp_plan& plan, const void* table_v, int64_t emb,
     const T* table = static_cast<const T*>(table_v);
     T* out = static_cast<T*>(out_v);
     T* partial = static_cast<T*>(scratch);
-    const Geometry geo = choose_geometry<T>(emb, {table, out, partial});
+    const Geometry geo = choose_geometry<T>(emb);
     return with_geometry<T>(geo, [&](auto vt, auto gt) -> int {
         constexpr int V = decltype(vt)::value;
         constexpr int G = decltype(gt)::value;
@@ -1465,7 +1613,7 @@ int segment_sum_scaled_t(const relm_mp_plan& plan, const void* table_v, int64_t 
     const T* base = static_cast<const T*>(base_v);
     T* out = static_cast<T*>(out_v);
     T* partial = static_cast<T*>(scratch);
-    const Geometry geo = choose_geometry<T>(emb, {table, base, out, partial});
+    const Geometry geo = choose_geometry<T>(emb);
     return with_geometry<T>(geo, [&](auto vt, auto gt) -> int {
         constexpr int V = decltype(vt)::value;
         constexpr int G = decltype(gt)::value;
@@ -1488,7 +1636,18 @@ int lse_backward_t(const relm_mp_plan& plan, const int64_t* gathers, const void*
     const T* rel = static_cast<const T*>(rel_v);
     T* grad_rel = static_cast<T*>(grad_rel_v);
     T* partial = static_cast<T*>(scratch);
-    const Geometry geo = choose_geometry<T>(emb, {grad_out, out, rel, grad_rel, partial});
+    if (plan.kind == RELM_MP_PLAN_INVERSE && flat_rows<T>(emb, plan.num_edges, plan.num_gather)) {
+        const auto flat = [&](auto src) {
+            hipLaunchKernelGGL((k_lse_bwd_flat<T, decltype(src)>), flat_grid<T>(plan.num_keys, emb), dim3(kThreads),
+                               0, s, plan.inv, plan.counts, plan.num_edges, src, plan.num_gather, grad_out, out, rel,
+                               plan.num_keys, static_cast<int32_t>(emb), flat_magic(emb), grad_rel,
+                               skip_on_collision);
+        };
+        if (snap != nullptr) flat(GathersSnap{snap->snap_keys, snap->snap_key_plain});
+        else flat(GathersI64{gathers});
+        return hip_error(hipGetLastError(), "relm_mp logsumexp backward kernel");
+    }
+    const Geometry geo = choose_geometry<T>(emb);
     return with_geometry<T>(geo, [&](auto vt, auto gt) -> int {
         constexpr int V = decltype(vt)::value;
         constexpr int G = decltype(gt)::value;
@@ -1553,7 +1712,7 @@ int segment_sum_msgdiv_t(const relm_mp_plan& plan, const void* table_v, int64_t 
     const T* base = static_cast<const T*>(base_v);
     T* out = static_cast<T*>(out_v);
     T* partial = static_cast<T*>(scratch);
-    const Geometry geo = choose_geometry<T>(emb, {table, base, out, partial});
+    const Geometry geo = choose_geometry<T>(emb);
     return with_geometry<T>(geo, [&](auto vt, auto gt) -> int {
         constexpr int V = decltype(vt)::value;
         constexpr int G = decltype(gt)::value;
@@ -1601,7 +1760,14 @@ int rows_scale_t(const void* in_v, const int64_t* gather, int div_kind, const in
     const T* in = static_cast<const T*>(in_v);
     const T* base = static_cast<const T*>(base_v);
     T* out = static_cast<T*>(out_v);
-    const Geometry geo = choose_geometry<T>(emb, {in, base, out});
+    Geometry geo = choose_geometry<T>(emb);
+    // in place, a column must not be read again after a second lane has written
+    // it: one element per lane where the lanes would share columns
+    if ((out == in || out == base) && emb % geo.V != 0) {
+        geo.V = 1;
+        geo.G = 64;
+        geo.slices = (emb + 63) / 64;
+    }
     return with_geometry<T>(geo, [&](auto vt, auto gt) -> int {
         constexpr int V = decltype(vt)::value;
         constexpr int G = decltype(gt)::value;
@@ -1708,7 +1874,7 @@ int sum_backward_edges_t(const relm_mp_plan& fwd, const relm_mp_plan_counts* cou
     const int64_t E = fwd.num_edges;
     const GathersSnap rows{fwd.snap_gathers, fwd.snap_gather_plain};
     const GathersSnap dsts{fwd.snap_keys, fwd.snap_key_plain};
-    const Geometry geo = choose_geometry<T>(emb, {grad_out, grad_rel});
+    const Geometry geo = choose_geometry<T>(emb);
     return with_geometry<T>(geo, [&](auto vt, auto gt) -> int {
         constexpr int V = decltype(vt)::value;
         constexpr int G = decltype(gt)::value;
@@ -1735,7 +1901,11 @@ int compute_backward_by_src(int dtype, const relm_mp_plan& dst_plan, const relm_
     // also reads every message row, keeps the rows in order: in edge order the
     // callers' layout reads and writes every other row per sweep (1.802
     // against 1.777 ms).
-    const bool by_edges = mode == RELM_MP_MODE_SUM && inv_plan.num_keys == dst_plan.num_edges;
+    // Rows that are no multiple of 16 bytes go through the map in flat pieces
+    // (k_gather_flat): in edge order they would be stored in parts of lines.
+    const bool flat = dtype == RELM_MP_F64 ? flat_rows<double>(emb, dst_plan.num_edges, dst_plan.num_keys)
+                                           : flat_rows<float>(emb, dst_plan.num_edges, dst_plan.num_keys);
+    const bool by_edges = mode == RELM_MP_MODE_SUM && inv_plan.num_keys == dst_plan.num_edges && !flat;
     const relm_mp_plan* snap = &dst_plan;
     if (mode == RELM_MP_MODE_SUM) {
         // as the edge-order sum backward: grad_out and the destinations read
