@@ -380,13 +380,20 @@ int inv_build(const int64_t* keys, int64_t key_bound, const char* key_name, cons
     plan->snap_key_plain = snap.key_plain;
     plan->snap_gathers = reinterpret_cast<const int32_t*>(snap.gathers);
     plan->snap_gather_plain = snap.gather_plain;
-    RELM_HIP(launch_status_init(l.status, s), "relm_mp status init");
-    RELM_HIP(launch_fill_i32(l.inv, key_bound, -1, s), "relm_mp fill");
-    RELM_HIP(launch_inv_build(keys, key_bound, gathers, gather_bound, num_edges, l.inv, snap,
-                              l.status, s),
-             "relm_mp inverse plan kernel");
     int32_t gen = 0;
-    RELM_HIP(hs->publish_status(l.status, l.counts, s, &gen), "relm_mp status publish");
+    if (small_plan(num_edges, key_bound)) {
+        const StatusPublish pub = hs->publish_target(l.status, &gen);
+        RELM_HIP(launch_inv_small(keys, key_bound, gathers, gather_bound, num_edges, l.inv, snap,
+                                  l.counts, l.status, pub, s),
+                 "relm_mp small inverse plan kernel");
+    } else {
+        RELM_HIP(launch_status_init(l.status, s), "relm_mp status init");
+        RELM_HIP(launch_fill_i32(l.inv, key_bound, -1, s), "relm_mp fill");
+        RELM_HIP(launch_inv_build(keys, key_bound, gathers, gather_bound, num_edges, l.inv, snap,
+                                  l.status, s),
+                 "relm_mp inverse plan kernel");
+        RELM_HIP(hs->publish_status(l.status, l.counts, s, &gen), "relm_mp status publish");
+    }
     if (!wait) {
         PendingCheck& p = hs->pending;
         p.active = true;
@@ -477,31 +484,41 @@ int csr_build(const int64_t* keys, int64_t key_bound, const char* key_name, cons
     plan->snap_gather_plain = gathers != nullptr ? l.snap_plain : nullptr;
     plan->max_degree = plan->num_hubs = plan->num_chunks = plan->num_multi_hubs = -1;
     plan->num_items = plan->num_short = -1;
-    const SortZero zero = sort_zero_region(sc.sort, num_edges);
-    RELM_HIP(launch_status_init(l.status, s, zero.p, zero.n), "relm_mp status init");
-    // The validation result is final after the first sort pass: the pass
-    // behind it publishes it to the host, and the rest of the build is
-    // enqueued before the host waits for it.
     int32_t status_gen = 0;
-    if (num_edges > 0) {
+    if (small_plan(num_edges, key_bound)) {
         const StatusPublish pub = hs != nullptr ? hs->publish_target(l.status, &status_gen) : StatusPublish{};
-        // short_gather is written by the key index after the sort: until
-        // then it holds the sort's intermediate keys
-        RELM_HIP(sort_by_key(keys, key_bound, gathers, gather_bound, num_edges, sc.sort,
-                             reinterpret_cast<uint32_t*>(l.short_gather),
-                             reinterpret_cast<uint32_t*>(l.gather_sorted), l.offsets, l.status, s,
-                             pub),
-                 "relm_mp radix sort");
+        const SmallCsr small{l.offsets, l.gather_sorted, l.hub_key, l.hub_chunk_base, l.multi_hubs,
+                             l.chunk_hub, l.item_first, l.item_short, l.num_items, l.short_off,
+                             l.short_gather, l.snap_keys, l.snap_gathers, l.snap_plain, l.counts};
+        RELM_HIP(launch_csr_small(keys, key_bound, gathers, gather_bound, num_edges, small, l.status,
+                                  pub, s),
+                 "relm_mp small CSR plan kernel");
     } else {
-        RELM_HIP(launch_fill_i32(l.offsets, key_bound + 1, 0, s), "relm_mp offsets fill");
-        if (hs != nullptr)
-            RELM_HIP(hs->publish_status(l.status, nullptr, s, &status_gen), "relm_mp status copy");
+        const SortZero zero = sort_zero_region(sc.sort, num_edges);
+        RELM_HIP(launch_status_init(l.status, s, zero.p, zero.n), "relm_mp status init");
+        // The validation result is final after the first sort pass: the pass
+        // behind it publishes it to the host, and the rest of the build is
+        // enqueued before the host waits for it.
+        if (num_edges > 0) {
+            const StatusPublish pub = hs != nullptr ? hs->publish_target(l.status, &status_gen) : StatusPublish{};
+            // short_gather is written by the key index after the sort: until
+            // then it holds the sort's intermediate keys
+            RELM_HIP(sort_by_key(keys, key_bound, gathers, gather_bound, num_edges, sc.sort,
+                                 reinterpret_cast<uint32_t*>(l.short_gather),
+                                 reinterpret_cast<uint32_t*>(l.gather_sorted), l.offsets, l.status, s,
+                                 pub),
+                     "relm_mp radix sort");
+        } else {
+            RELM_HIP(launch_fill_i32(l.offsets, key_bound + 1, 0, s), "relm_mp offsets fill");
+            if (hs != nullptr)
+                RELM_HIP(hs->publish_status(l.status, nullptr, s, &status_gen), "relm_mp status copy");
+        }
+        RELM_HIP(launch_key_index(l.offsets, l.gather_sorted, key_bound, sc.key_index, l.hub_key,
+                                  l.hub_chunk_base, l.multi_hubs, l.chunk_hub, max_hubs(num_edges),
+                                  max_chunks(num_edges), l.item_first, l.item_short, l.num_items,
+                                  l.short_off, l.short_gather, l.counts, l.status, s),
+                 "relm_mp key index kernels");
     }
-    RELM_HIP(launch_key_index(l.offsets, l.gather_sorted, key_bound, sc.key_index, l.hub_key,
-                              l.hub_chunk_base, l.multi_hubs, l.chunk_hub, max_hubs(num_edges),
-                              max_chunks(num_edges), l.item_first, l.item_short, l.num_items,
-                              l.short_off, l.short_gather, l.counts, l.status, s),
-             "relm_mp key index kernels");
     DevStatus host{};
     if (hs != nullptr) {
         RELM_TRY(wait_host_word(hs->status_gen, status_gen, s, "relm_mp status wait"));

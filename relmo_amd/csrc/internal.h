@@ -147,6 +147,37 @@ hipError_t launch_key_index(const int32_t* offsets, const int32_t* gather_sorted
                             int64_t item_capacity, int32_t* short_off, int32_t* short_gather,
                             relm_mp_plan_counts* counts, DevStatus* st, hipStream_t s);
 
+// ---- plans of small inputs (small_plan_kernels.hip) -------------------------
+// Edges and keys that one workgroup's LDS takes.
+constexpr int kSmallPlanMax = 16384;
+bool small_plan(int64_t num_edges, int64_t num_keys);
+// The arrays of a CSR plan (relm_mp_plan), as csr_layout carves them.
+struct SmallCsr {
+    int32_t* offsets;
+    int32_t* gather_sorted;
+    int32_t* hub_key;
+    int32_t* hub_chunk_base;
+    int32_t* multi_hubs;
+    int32_t* chunk_hub;
+    int32_t* item_first;
+    int32_t* item_short;
+    int64_t item_capacity;
+    int32_t* short_off;
+    int32_t* short_gather;
+    uint32_t* snap_keys;
+    uint32_t* snap_gathers;
+    uint32_t* snap_plain;
+    relm_mp_plan_counts* counts;
+};
+// The whole build of a plan for which small_plan holds, the status included.
+hipError_t launch_csr_small(const int64_t* keys, int64_t key_bound, const int64_t* gathers,
+                            int64_t gather_bound, int64_t n, const SmallCsr& a, DevStatus* st,
+                            const StatusPublish& pub, hipStream_t s);
+hipError_t launch_inv_small(const int64_t* keys, int64_t key_bound, const int64_t* gathers,
+                            int64_t gather_bound, int64_t n, int32_t* inv, const SnapOut& snap,
+                            relm_mp_plan_counts* counts, DevStatus* st, const StatusPublish& pub,
+                            hipStream_t s);
+
 // Capacities of the hub arrays of a CSR plan over num_edges edges.
 inline int64_t max_hubs(int64_t num_edges) { return num_edges / (kHubThreshold + 1) + 1; }
 inline int64_t max_chunks(int64_t num_edges) {

@@ -1,0 +1,126 @@
+"""Plans of small inputs, built by one workgroup in one launch: every array of
+the CSR plan and the inverse map against the oracle's stable order, around the
+sizes where the kernels change (waves, rounds, the two capacities, one and two
+sort passes) and just past them, where the general kernels build the same."""
+
+from __future__ import annotations
+
+import re
+from pathlib import Path
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+ITEM = int(re.search(r"#define RELM_MP_ITEM_SIZE (\d+)",
+                     (Path(__file__).parent.parent / "include" / "relm_mp.h").read_text()).group(1))
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU visible")
+
+
+def _t(a: np.ndarray) -> torch.Tensor:
+    return torch.from_numpy(a).to(DEV)
+
+
+def _np(t: torch.Tensor) -> np.ndarray:
+    return t.cpu().numpy()
+
+
+def _arr(bp, name: str, n: int) -> np.ndarray:
+    return _np(bp._i32(getattr(bp.plan, name), n)) if n else np.zeros(0, np.int32)
+
+
+@pytest.mark.parametrize("num_keys,num_edges", [
+    (1, 1), (1, 16384), (2, 63), (7, 64), (128, 65), (129, 1023), (4096, 1024), (200, 3200), (4096, 4096),
+    (4097, 4096), (300, 4097), (16384, 5), (16384, 16384), (16383, 16321), (1000, 12289), (16385, 100),
+    (100, 16385),
+])
+@pytest.mark.parametrize("form", ["none", "identity", "permuted", "skewed"])
+def test_small_plans_against_the_oracle(num_keys: int, num_edges: int, form: str) -> None:
+    from relmo_amd import capi
+
+    print(f"small plan keys={num_keys} edges={num_edges} {form}", flush=True)
+    rng = np.random.default_rng(num_keys * 31 + num_edges)
+    if form == "skewed":  # hubs of one and of several chunks
+        keys = np.minimum(rng.pareto(0.5, num_edges).astype(np.int64), num_keys - 1)
+    else:
+        keys = rng.integers(0, num_keys, num_edges)
+    rows = num_edges + 3
+    if form == "none":
+        gathers = None
+    elif form == "identity":
+        gathers = np.arange(num_edges)
+    else:  # the second snapshot tile holds its own edge ids
+        gathers = rng.integers(0, rows, num_edges)
+        gathers[4096:8192] = np.arange(num_edges)[4096:8192]
+    kt, gt = _t(keys), None if gathers is None else _t(gathers)
+    msgs = np.arange(num_edges) if gathers is None else gathers
+
+    bp = capi.csr_plan(kt, num_keys, gt, num_edges if gathers is None else rows)
+    offsets, perm = oracle.csr_build(keys, num_keys)
+    assert np.array_equal(_np(bp.offsets), offsets)
+    assert np.array_equal(_np(bp.gather_sorted), msgs[perm])
+    deg = np.diff(offsets)
+    hub = deg > bp.plan.hub_threshold
+    chunks = np.where(hub, -(-deg // bp.plan.chunk_size), 0)
+    counts = (deg.max(), hub.sum(), chunks.sum(), (chunks > 1).sum())
+    assert (bp.plan.max_degree, bp.plan.num_hubs, bp.plan.num_chunks, bp.plan.num_multi_hubs) == counts
+    assert bp.plan.gather_identity == int(np.array_equal(msgs, np.arange(num_edges)))
+    hubs = np.flatnonzero(hub)
+    assert np.array_equal(_arr(bp, "hub_key", hubs.size), hubs)
+    assert np.array_equal(_arr(bp, "hub_chunk_base", hubs.size), (np.cumsum(chunks) - chunks)[hubs])
+    assert np.array_equal(_arr(bp, "chunk_hub", int(chunks.sum())), np.repeat(np.arange(hubs.size), chunks[hubs]))
+    assert np.array_equal(_arr(bp, "multi_hubs", int((chunks > 1).sum())), np.flatnonzero(chunks[hubs] > 1))
+    short = np.where(hub, 0, deg)
+    W = np.concatenate([[0], np.cumsum(1 + short)])
+    assert bp.plan.num_items == W[-1] // ITEM + 1
+    items = np.append(np.searchsorted(W[:-1], np.arange(bp.plan.num_items) * ITEM, side="left"), num_keys)
+    assert np.array_equal(_np(bp.item_first), items)
+    short_off = W - np.arange(num_keys + 1)
+    assert np.array_equal(_np(bp.short_off), short_off)
+    assert np.array_equal(_np(bp.item_short), short_off[items])
+    assert bp.plan.num_short == int(short.sum())
+    assert np.array_equal(_np(bp.short_gather), msgs[perm][~np.repeat(hub, deg)])
+
+    inv = capi.inv_plan(kt, num_keys, gt, rows, snapshot=True)
+    want, collisions = oracle.inverse_build(keys, num_keys)
+    assert np.array_equal(_np(inv.inv), want)
+    assert inv.plan.collisions == collisions
+
+    # the snapshots: the same indices match, one changed index (the last) does not
+    for plan in (bp, inv):
+        assert capi.plan_match(kt, gt, [plan]) == [True]
+        other = keys.copy()
+        other[-1] += 1
+        assert capi.plan_match(_t(other), gt, [plan]) == [False]
+
+    # bad indices: the smallest bad edge of each array is the one reported
+    if num_edges >= 3:
+        bad = keys.copy()
+        bad[num_edges // 3], bad[-1] = num_keys + 5, -2
+        for build in (capi.csr_plan, capi.inv_plan):
+            with pytest.raises((RuntimeError, ValueError), match=rf"key index out of bounds: {num_keys + 5} not in"):
+                build(_t(bad), num_keys, gt, rows)
+        if gathers is not None:
+            bad_g = gathers.copy()
+            bad_g[num_edges // 2], bad_g[-1] = -1, rows
+            for build in (capi.csr_plan, capi.inv_plan):
+                with pytest.raises((RuntimeError, ValueError), match="gather index out of bounds: -1 not in"):
+                    build(kt, num_keys, _t(bad_g), rows)
+
+
+def test_small_identity_inverse() -> None:
+    from relmo_amd import capi
+
+    for n, keys in ((1, 1), (4096, 4097), (10_000, 16_384)):
+        bp = capi.inv_plan(_t(np.arange(n)), keys, None, 0)
+        assert not bp.plan.inv and bp.plan.collisions == 0
