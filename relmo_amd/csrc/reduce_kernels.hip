@@ -998,154 +998,101 @@ __global__ __launch_bounds__(kThreads) void k_gather_inv(const int32_t* __restri
     }
 }
 
-// Rows whose size is no multiple of 16 bytes: the output as one flat array in
-// aligned pieces of 16 bytes, each the end of one row and the start of the next
-// where it lies across their seam.  Every lane stores a whole piece, so the
-// stores fill whole lines; a row to a row group stores pieces of lines that its
-// neighbours complete later: the sum backward of 3 M messages of 33 floats takes
-// 180 us in pieces, 278 us by rows in 4-byte lanes and 309 in 16-byte ones.  A
-// thread keeps kFlatPieces pieces in flight.
-constexpr int kFlatPieces = 4;
-constexpr int64_t kFlatMaxColumns = 4096;  // n / D below by one 32-bit multiply: n < D + 4096, both below 2^16
+// Rows whose size is no multiple of 16 bytes: the output as one flat array of
+// units of V elements, V the widest that divides the row (8 bytes at even widths
+// of floats, else one element).  Neighbouring lanes take neighbouring units
+// across row seams, so every lane works whatever the width and a wave stores one
+// contiguous range; loads and stores keep their natural alignment, which a
+// 16-byte piece at an odd place does not (each then costs two).  Backward of 4.2
+// M messages of 30 floats on 145,216 keys: 125 us by units, 151 by rows in 8-byte
+// lanes, 220 in 16-byte pieces across the seams; its logsumexp step 548, 560 and
+// 774 us.  A thread keeps UNITS units in flight, kThreads apart (4 and 16 were
+// up to 8% slower than 8 for the gather).
+constexpr int kGatherUnits = 8;
+constexpr int kLseUnits = 4;
+constexpr int64_t kUnitsMaxRow = 16384;  // n / units_per_row below by one 32-bit multiply: n < 2^16
 
-template <int V>
-struct FlatPiece {
-    int64_t at;    // first element in the output
-    int64_t left;  // elements of the output from there on, <= 0 past its end
-    int col;       // column of the first element
-    int over;      // elements that belong to the next row
+template <int UNITS>
+struct UnitRows {
+    InvRow r[UNITS];
+    uint32_t col[UNITS];  // unit of the row
+    // The units [f0, f0 + kThreads * UNITS) of this workgroup: unit j of the
+    // thread is f0 + j * kThreads + threadIdx.x.
+    __device__ __forceinline__ UnitRows(int64_t f0, int64_t num_keys, uint32_t units_per_row, uint32_t magic) {
+        const int64_t row0 = f0 / units_per_row;
+        const uint32_t rem = static_cast<uint32_t>(f0 - row0 * units_per_row);
+#pragma unroll
+        for (int j = 0; j < UNITS; ++j) {
+            const uint32_t o = rem + static_cast<uint32_t>(j * kThreads) + threadIdx.x;
+            const uint32_t q = __umulhi(o, magic);
+            col[j] = o - q * units_per_row;
+            r[j].live = row0 + q < num_keys;
+            r[j].key = r[j].live ? row0 + q : 0;
+        }
+    }
 };
 
-// Pieces of this thread in the chunk of kThreads * kFlatPieces * V elements at
-// f0, and their rows: r[2 j] the first row of piece j, r[2 j + 1] the second
-// (the first again where the piece lies in one row).
-template <int V>
-__device__ __forceinline__ void flat_pieces(FlatPiece<V> (&p)[kFlatPieces], InvRow (&r)[2 * kFlatPieces],
-                                            int64_t f0, int64_t num_keys, int32_t D, uint32_t magic) {
-    const int64_t row0 = f0 / D;
-    const uint32_t rem = static_cast<uint32_t>(f0 - row0 * D);
-    const int64_t total = num_keys * D;
-#pragma unroll
-    for (int j = 0; j < kFlatPieces; ++j) {
-        const uint32_t o = static_cast<uint32_t>(j * kThreads + static_cast<int>(threadIdx.x)) * V;
-        const uint32_t q = __umulhi(rem + o, magic);
-        p[j].at = f0 + o;
-        p[j].left = total - p[j].at;
-        p[j].col = static_cast<int>(rem + o - q * static_cast<uint32_t>(D));
-        p[j].over = max(p[j].col + V - D, 0);
-        const int64_t row = row0 + q;
-        const bool two = p[j].over > 0 && row + 1 < num_keys;
-        r[2 * j].live = r[2 * j + 1].live = row < num_keys;
-        r[2 * j].key = row < num_keys ? row : 0;
-        r[2 * j + 1].key = r[2 * j].key + (two ? 1 : 0);
-    }
-}
-
-// The V elements from column `col` of table row a and on into row b: row a's
-// last V elements, and row b's first ones moved in behind them.
-template <typename T, int V>
-__device__ __forceinline__ Pack<T, V> flat_load(const T* __restrict__ table, int64_t D, const InvRow& a,
-                                                const InvRow& b, int col, int over) {
-    const Pack<T, V> x = pack_load<T, V>(table + row_offset(a.g, D) + (col - over));
-    Pack<T, V> y = x;
-    if (over > 0) y = pack_load<T, V>(table + row_offset(b.g, D));
-    T w[2 * V];
-#pragma unroll
-    for (int i = 0; i < V; ++i) {
-        w[i] = a.ok ? x.v[i] : T(0);
-        w[V + i] = b.ok ? y.v[i] : T(0);
-    }
-#pragma unroll
-    for (int s = 1; s < V; s *= 2) {
-        const bool shift = (over & s) != 0;
-#pragma unroll
-        for (int i = 0; i + s < 2 * V; ++i) w[i] = shift ? w[i + s] : w[i];
-    }
-    Pack<T, V> v;
-#pragma unroll
-    for (int i = 0; i < V; ++i) v.v[i] = w[i];
-    return v;
-}
-
-template <typename T, int V>
-__device__ __forceinline__ void flat_store(T* __restrict__ out, const FlatPiece<V>& p, const Pack<T, V>& v) {
-    if (p.left >= V) {
-        pack_store_stream<T, V>(out + p.at, v);
-    } else {
-#pragma unroll
-        for (int i = 0; i < V; ++i)
-            if (i < p.left) out[p.at + i] = v.v[i];
-    }
-}
-
-// k_gather_inv by flat pieces (V < D <= kFlatMaxColumns).
-template <typename T, class Src>
-__global__ __launch_bounds__(kThreads) void k_gather_flat(const int32_t* __restrict__ inv_in,
-                                                          const relm_mp_plan_counts* __restrict__ pc,
-                                                          int64_t num_edges, Src gathers, int64_t num_gather,
-                                                          const T* __restrict__ table, int64_t num_keys,
-                                                          int32_t D, uint32_t magic, T* __restrict__ out,
-                                                          bool skip_on_collision) {
-    constexpr int V = 16 / static_cast<int>(sizeof(T));
-    constexpr int64_t kChunk = static_cast<int64_t>(kThreads) * kFlatPieces * V;
-    if (skip_on_collision && pc->collisions != 0) return;
-    const int32_t* inv = inverse_map(inv_in, pc);
-    for (int64_t f0 = blockIdx.x * kChunk; f0 < num_keys * D; f0 += gridDim.x * kChunk) {
-        FlatPiece<V> p[kFlatPieces];
-        InvRow r[2 * kFlatPieces];
-        flat_pieces<V>(p, r, f0, num_keys, D, magic);
-        inverse_gather(r, inv, num_edges, gathers, num_gather);
-        Pack<T, V> v[kFlatPieces];
-#pragma unroll
-        for (int j = 0; j < kFlatPieces; ++j)
-            v[j] = flat_load<T, V>(table, D, r[2 * j], r[2 * j + 1], p[j].col, p[j].over);
-#pragma unroll
-        for (int j = 0; j < kFlatPieces; ++j) flat_store<T, V>(out, p[j], v[j]);
-    }
-}
-
-// k_lse_bwd_inv by flat pieces.
-template <typename T, class Src>
-__global__ __launch_bounds__(kThreads) void k_lse_bwd_flat(const int32_t* __restrict__ inv_in,
+// k_gather_inv by units.
+template <typename T, int V, class Src>
+__global__ __launch_bounds__(kThreads) void k_gather_units(const int32_t* __restrict__ inv_in,
                                                            const relm_mp_plan_counts* __restrict__ pc,
                                                            int64_t num_edges, Src gathers, int64_t num_gather,
-                                                           const T* __restrict__ grad_out,
-                                                           const T* __restrict__ out, const T* __restrict__ rel,
-                                                           int64_t num_keys, int32_t D, uint32_t magic,
-                                                           T* __restrict__ grad_rel, bool skip_on_collision) {
-    constexpr int V = 16 / static_cast<int>(sizeof(T));
-    constexpr int64_t kChunk = static_cast<int64_t>(kThreads) * kFlatPieces * V;
+                                                           const T* __restrict__ table, int64_t num_keys,
+                                                           uint32_t units_per_row, uint32_t magic,
+                                                           T* __restrict__ out, bool skip_on_collision) {
+    constexpr int64_t kChunk = static_cast<int64_t>(kThreads) * kGatherUnits;
     if (skip_on_collision && pc->collisions != 0) return;
     const int32_t* inv = inverse_map(inv_in, pc);
-    for (int64_t f0 = blockIdx.x * kChunk; f0 < num_keys * D; f0 += gridDim.x * kChunk) {
-        FlatPiece<V> p[kFlatPieces];
-        InvRow r[2 * kFlatPieces];
-        flat_pieces<V>(p, r, f0, num_keys, D, magic);
-        inverse_gather(r, inv, num_edges, gathers, num_gather);
-        Pack<T, V> x[kFlatPieces], g[kFlatPieces], o[kFlatPieces];
+    for (int64_t f0 = blockIdx.x * kChunk; f0 < num_keys * units_per_row; f0 += gridDim.x * kChunk) {
+        UnitRows<kGatherUnits> u(f0, num_keys, units_per_row, magic);
+        inverse_gather(u.r, inv, num_edges, gathers, num_gather);
+        Pack<T, V> v[kGatherUnits];
 #pragma unroll
-        for (int j = 0; j < kFlatPieces; ++j) {
-            // the last piece may end behind the rows: read one that does not
-            const int64_t back = p[j].left >= V ? 0 : V - p[j].left;
-            x[j] = pack_load_stream<T, V>(rel + (p[j].left > 0 ? p[j].at - back : 0));
-            if (p[j].left > 0 && back > 0) {
+        for (int j = 0; j < kGatherUnits; ++j)
+            v[j] = pack_load<T, V>(table + (row_offset(u.r[j].g, units_per_row) + u.col[j]) * V);
 #pragma unroll
-                for (int i = 0; i < V; ++i) x[j].v[i] = rel[i < p[j].left ? p[j].at + i : p[j].at];
-            }
-            g[j] = flat_load<T, V>(grad_out, D, r[2 * j], r[2 * j + 1], p[j].col, p[j].over);
-            o[j] = flat_load<T, V>(out, D, r[2 * j], r[2 * j + 1], p[j].col, p[j].over);
+        for (int j = 0; j < kGatherUnits; ++j) {
+            if (!u.r[j].ok) v[j] = pack_fill<T, V>(T(0));
+            if (u.r[j].live) pack_store_stream<T, V>(out + (f0 + j * kThreads + threadIdx.x) * V, v[j]);
+        }
+    }
+}
+
+// k_lse_bwd_inv by units.
+template <typename T, int V, class Src>
+__global__ __launch_bounds__(kThreads) void k_lse_bwd_units(const int32_t* __restrict__ inv_in,
+                                                            const relm_mp_plan_counts* __restrict__ pc,
+                                                            int64_t num_edges, Src gathers, int64_t num_gather,
+                                                            const T* __restrict__ grad_out,
+                                                            const T* __restrict__ out, const T* __restrict__ rel,
+                                                            int64_t num_keys, uint32_t units_per_row,
+                                                            uint32_t magic, T* __restrict__ grad_rel,
+                                                            bool skip_on_collision) {
+    constexpr int64_t kChunk = static_cast<int64_t>(kThreads) * kLseUnits;
+    if (skip_on_collision && pc->collisions != 0) return;
+    const int32_t* inv = inverse_map(inv_in, pc);
+    for (int64_t f0 = blockIdx.x * kChunk; f0 < num_keys * units_per_row; f0 += gridDim.x * kChunk) {
+        UnitRows<kLseUnits> u(f0, num_keys, units_per_row, magic);
+        Pack<T, V> x[kLseUnits], g[kLseUnits], o[kLseUnits];
+#pragma unroll
+        for (int j = 0; j < kLseUnits; ++j)
+            x[j] = pack_load_stream<T, V>(rel + (u.r[j].live ? f0 + j * kThreads + threadIdx.x : 0) * V);
+        inverse_gather(u.r, inv, num_edges, gathers, num_gather);
+#pragma unroll
+        for (int j = 0; j < kLseUnits; ++j) {
+            const uint64_t at = (row_offset(u.r[j].g, units_per_row) + u.col[j]) * V;
+            g[j] = pack_load<T, V>(grad_out + at);
+            o[j] = pack_load<T, V>(out + at);
         }
 #pragma unroll
-        for (int j = 0; j < kFlatPieces; ++j) {
+        for (int j = 0; j < kLseUnits; ++j) {
             Pack<T, V> res;
 #pragma unroll
             for (int i = 0; i < V; ++i) {
-                const bool ok = i < V - p[j].over ? r[2 * j].ok : r[2 * j + 1].ok;
-                const T w = fast_exp<T>(x[j].v[i] - o[j].v[i]);
-                const T c = g[j].v[i] * w;
-                res.v[i] = ok ? T(0) + c : T(0);
+                const T c = g[j].v[i] * fast_exp<T>(x[j].v[i] - o[j].v[i]);
+                res.v[i] = u.r[j].ok ? T(0) + c : T(0);
             }
-            flat_store<T, V>(grad_rel, p[j], res);
+            if (u.r[j].live) pack_store_stream<T, V>(grad_rel + (f0 + j * kThreads + threadIdx.x) * V, res);
         }
     }
 }
@@ -1373,17 +1320,20 @@ struct Geometry {
 
 // 16 bytes per lane whatever the alignment (lane_column), one element where a
 // row has fewer.  Narrower lanes where the rows or the base are not aligned cost
-// more than the straddled lines do: 2 M argument slots of 128 floats at an
+// the reductions more than the straddled lines do: 2 M argument slots of 128 floats at an
 // 8-byte aligned column 575 us in 8-byte lanes, 503 in 16-byte ones; the hub
 // chunks of 3 M messages of 33 floats 120 us in 4-byte lanes, 106 in 16-byte ones.
-template <typename T>
-Geometry choose_geometry(int64_t D) {
-    constexpr int kVecMax = 16 / static_cast<int>(sizeof(T));
-    const int V = D >= kVecMax ? kVecMax : 1;
+inline Geometry lanes_geometry(int64_t D, int V) {
     const int64_t vcols = (D + V - 1) / V;
     int G = 4;
     while (G < vcols && G < 64) G *= 2;
     return {V, G, (vcols + G - 1) / G};
+}
+
+template <typename T>
+Geometry choose_geometry(int64_t D) {
+    constexpr int kVecMax = 16 / static_cast<int>(sizeof(T));
+    return lanes_geometry(D, D >= kVecMax ? kVecMax : 1);
 }
 
 template <typename T, typename F>
@@ -1412,21 +1362,33 @@ dim3 row_grid(int64_t rows, int G, int64_t slices, int rows_per_group = 1) {
     return dim3(static_cast<unsigned>(bx), static_cast<unsigned>(slices));
 }
 
-// Whether rows of D elements go through the flat kernels.
+// Elements of a unit of a row of D elements (k_gather_units), or 0 where the row
+// kernels take it: rows of whole 16-byte lanes, of one unit, and those too long
+// for the units' division.
 template <typename T>
-bool flat_rows(int64_t D, int64_t num_edges, int64_t num_gather) {
-    constexpr int V = 16 / static_cast<int>(sizeof(T));
-    return D > V && D % V != 0 && D <= kFlatMaxColumns && num_edges > 0 && num_gather > 0;
+int unit_width(int64_t D, int64_t num_edges, int64_t num_gather) {
+    constexpr int kVecMax = 16 / static_cast<int>(sizeof(T));
+    if (D % kVecMax == 0 || num_edges <= 0 || num_gather <= 0) return 0;
+    const int V = kVecMax > 2 && D > 2 && D % 2 == 0 ? 2 : 1;
+    return D / V > 1 && D / V <= kUnitsMaxRow ? V : 0;
 }
 
-template <typename T>
-dim3 flat_grid(int64_t rows, int64_t D) {
-    constexpr int64_t kChunk = static_cast<int64_t>(kThreads) * kFlatPieces * (16 / sizeof(T));
-    return dim3(static_cast<unsigned>(std::min<int64_t>((rows * D + kChunk - 1) / kChunk, kMaxBlocksX)));
+dim3 unit_grid(int64_t units, int per_thread) {
+    const int64_t chunk = static_cast<int64_t>(kThreads) * per_thread;
+    return dim3(static_cast<unsigned>(std::min<int64_t>((units + chunk - 1) / chunk, kMaxBlocksX)));
 }
 
-// ceil(2^32 / D): n / D = high word of n * magic for n, D < 2^16.
-uint32_t flat_magic(int64_t D) { return static_cast<uint32_t>(((uint64_t(1) << 32) + D - 1) / D); }
+// ceil(2^32 / d): n / d = high word of n * magic for n, d < 2^16 (d > 1).
+uint32_t unit_magic(int64_t d) { return static_cast<uint32_t>(((uint64_t(1) << 32) + d - 1) / d); }
+
+// Calls f(std::integral_constant<int, V>) for a unit width V.
+template <typename T, typename F>
+int with_unit(int V, F&& f) {
+    if constexpr (sizeof(T) < 8) {
+        if (V == 2) return f(std::integral_constant<int, 2>{});
+    }
+    return f(std::integral_constant<int, 1>{});
+}
 
 // Workgroups of `kernel` (kThreads each) resident on the current device at
 // once; persistent launches size their grids with it.
@@ -1544,15 +1506,28 @@ int gather_last_t(const relm_mp_plan& plan, const int64_t* gathers, const void* 
         return with_geometry<T>(
             geo, [&](auto vt, auto gt) -> int { return launch(vt, gt, geo, rows); });
     }
-    if (plan.kind == RELM_MP_PLAN_INVERSE && flat_rows<T>(emb, plan.num_edges, plan.num_gather)) {
-        const auto flat = [&](auto src) {
-            hipLaunchKernelGGL((k_gather_flat<T, decltype(src)>), flat_grid<T>(plan.num_keys, emb), dim3(kThreads), 0,
-                               s, plan.inv, plan.counts, plan.num_edges, src, plan.num_gather, table,
-                               plan.num_keys, static_cast<int32_t>(emb), flat_magic(emb), out, skip_on_collision);
-        };
-        if (snap != nullptr) flat(GathersSnap{snap->snap_keys, snap->snap_key_plain});
-        else flat(GathersI64{gathers});
-        return hip_error(hipGetLastError(), "relm_mp gather kernel");
+    const int unit = plan.kind == RELM_MP_PLAN_INVERSE ? unit_width<T>(emb, plan.num_edges, plan.num_gather) : 0;
+    // Rows of an odd width that leave at most one lane in 32 idle (31, 63, 127
+    // floats): one element per lane, where a row's index is read once and not
+    // once per unit - 4 M rows of 31 366 us against 391, 2 M of 63 472 against 491.
+    const Geometry single = lanes_geometry(emb, 1);
+    if (unit == 1 && 32 * emb >= 31 * single.G * single.slices)
+        return with_geometry<T>(
+            single, [&](auto vt, auto gt) -> int { return launch(vt, gt, single, DenseRows{}); });
+    if (unit > 0) {
+        return with_unit<T>(unit, [&](auto vt) -> int {
+            constexpr int V = decltype(vt)::value;
+            const int64_t per_row = emb / V;
+            const auto go = [&](auto src) {
+                hipLaunchKernelGGL((k_gather_units<T, V, decltype(src)>), unit_grid(plan.num_keys * per_row, kGatherUnits),
+                                   dim3(kThreads), 0, s, plan.inv, plan.counts, plan.num_edges, src, plan.num_gather,
+                                   table, plan.num_keys, static_cast<uint32_t>(per_row), unit_magic(per_row), out,
+                                   skip_on_collision);
+            };
+            if (snap != nullptr) go(GathersSnap{snap->snap_keys, snap->snap_key_plain});
+            else go(GathersI64{gathers});
+            return hip_error(hipGetLastError(), "relm_mp gather kernel");
+        });
     }
     const Geometry geo = choose_geometry<T>(emb);
     return with_geometry<T>(geo,
@@ -1636,16 +1611,21 @@ int lse_backward_t(const relm_mp_plan& plan, const int64_t* gathers, const void*
     const T* rel = static_cast<const T*>(rel_v);
     T* grad_rel = static_cast<T*>(grad_rel_v);
     T* partial = static_cast<T*>(scratch);
-    if (plan.kind == RELM_MP_PLAN_INVERSE && flat_rows<T>(emb, plan.num_edges, plan.num_gather)) {
-        const auto flat = [&](auto src) {
-            hipLaunchKernelGGL((k_lse_bwd_flat<T, decltype(src)>), flat_grid<T>(plan.num_keys, emb), dim3(kThreads),
-                               0, s, plan.inv, plan.counts, plan.num_edges, src, plan.num_gather, grad_out, out, rel,
-                               plan.num_keys, static_cast<int32_t>(emb), flat_magic(emb), grad_rel,
-                               skip_on_collision);
-        };
-        if (snap != nullptr) flat(GathersSnap{snap->snap_keys, snap->snap_key_plain});
-        else flat(GathersI64{gathers});
-        return hip_error(hipGetLastError(), "relm_mp logsumexp backward kernel");
+    const int unit = plan.kind == RELM_MP_PLAN_INVERSE ? unit_width<T>(emb, plan.num_edges, plan.num_gather) : 0;
+    if (unit > 0) {
+        return with_unit<T>(unit, [&](auto vt) -> int {
+            constexpr int V = decltype(vt)::value;
+            const int64_t per_row = emb / V;
+            const auto go = [&](auto src) {
+                hipLaunchKernelGGL((k_lse_bwd_units<T, V, decltype(src)>), unit_grid(plan.num_keys * per_row, kLseUnits),
+                                   dim3(kThreads), 0, s, plan.inv, plan.counts, plan.num_edges, src, plan.num_gather,
+                                   grad_out, out, rel, plan.num_keys, static_cast<uint32_t>(per_row),
+                                   unit_magic(per_row), grad_rel, skip_on_collision);
+            };
+            if (snap != nullptr) go(GathersSnap{snap->snap_keys, snap->snap_key_plain});
+            else go(GathersI64{gathers});
+            return hip_error(hipGetLastError(), "relm_mp logsumexp backward kernel");
+        });
     }
     const Geometry geo = choose_geometry<T>(emb);
     return with_geometry<T>(geo, [&](auto vt, auto gt) -> int {
@@ -1901,11 +1881,11 @@ int compute_backward_by_src(int dtype, const relm_mp_plan& dst_plan, const relm_
     // also reads every message row, keeps the rows in order: in edge order the
     // callers' layout reads and writes every other row per sweep (1.802
     // against 1.777 ms).
-    // Rows that are no multiple of 16 bytes go through the map in flat pieces
-    // (k_gather_flat): in edge order they would be stored in parts of lines.
-    const bool flat = dtype == RELM_MP_F64 ? flat_rows<double>(emb, dst_plan.num_edges, dst_plan.num_keys)
-                                           : flat_rows<float>(emb, dst_plan.num_edges, dst_plan.num_keys);
-    const bool by_edges = mode == RELM_MP_MODE_SUM && inv_plan.num_keys == dst_plan.num_edges && !flat;
+    // Rows that are no multiple of 16 bytes go through the map in units
+    // (k_gather_units): in edge order they would be stored in parts of lines.
+    const bool units = (dtype == RELM_MP_F64 ? unit_width<double>(emb, dst_plan.num_edges, dst_plan.num_keys)
+                                             : unit_width<float>(emb, dst_plan.num_edges, dst_plan.num_keys)) > 0;
+    const bool by_edges = mode == RELM_MP_MODE_SUM && inv_plan.num_keys == dst_plan.num_edges && !units;
     const relm_mp_plan* snap = &dst_plan;
     if (mode == RELM_MP_MODE_SUM) {
         // as the edge-order sum backward: grad_out and the destinations read
