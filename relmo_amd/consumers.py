@@ -671,9 +671,9 @@ class CentralizedRelationalGNN(nn.Module):
     def _hidden_pad(self, t: Tensor, r: dict) -> int:
         """Zero columns appended to the hidden width on the fused path (one
         hidden layer) to make it a multiple of 4: rows of 398 floats are only
-        8-byte aligned, rows of 400 take 16-byte lanes in the gathers and the
-        FiLM kernels (C5: a 398-wide gather-sum of 10.8 M rows 5.4 ms, 400-wide
-        3.9 ms).  The padding columns stay exactly zero through the Linear
+        8-byte aligned, rows of 400 start and end on 16 bytes (a 398-wide
+        gather-sum of 10.8 M rows in 8-byte lanes 5.4 ms, 400-wide in 16-byte
+        lanes 3.9 ms).  The padding columns stay exactly zero through the Linear
         (zero weight rows and bias), FiLM (zero gamma and beta: mish(0) = 0)
         and the output Linear (zero weight columns); F.pad's backward drops
         their gradients."""

@@ -37,9 +37,8 @@ namespace {
 constexpr int kThreads = 256;
 // Rows per row group per iteration of the inverse-plan row kernels, the best
 // of 1..8 measured: the gather of 16-byte lanes (C3, D = 64; edge order,
-// D = 32) keeps 2 rows in flight, of narrower lanes (argument slots of 128
-// columns at an 8-byte aligned offset) 8; the logsumexp backward, which
-// reads three rows per row, 4.
+// D = 32) keeps 2 rows in flight, of narrower lanes 8; the logsumexp backward,
+// which reads three rows per row, 4.
 template <typename T, int V>
 constexpr int gather_rows_in_flight() { return sizeof(T) * V >= 16 ? 2 : 8; }
 constexpr int kLseRowsInFlight = 4;

@@ -1,7 +1,7 @@
 """Row widths that are no multiple of 16 bytes, through the public ops: rows
 whose last lane shares columns with the one before it (the CSR reductions) and
-outputs written in 16-byte pieces across row seams (the inverse-plan gathers
-and the logsumexp backward), against torch in float64."""
+outputs written in 8- or 4-byte units across row seams (the inverse-plan
+gathers and the logsumexp backward), against torch in float64."""
 
 from __future__ import annotations
 
