@@ -348,10 +348,16 @@ __global__ __launch_bounds__(kThreads) void k_inv_small(
     if (bad_g != ~0u) atomicMin(&s_bad[1], bad_g);
     if (lost != 0) atomicAdd(&s_lost, lost);
     __syncthreads();
+    for (int k = tid; k < nk; k += kThreads) inv[k] = s_inv[k];
     if (tid < (n + kSnapTile - 1) / kSnapTile) {
         if (snap.key_plain != nullptr) snap.key_plain[tid] = s_mis[tid] != 0u ? 0u : 1u;
         if (snap.gather_plain != nullptr) snap.gather_plain[tid] = s_mis[kTiles + tid] != 0u ? 0u : 1u;
     }
+    // Published behind the whole plan, as by the general build: the host's word
+    // is all that a caller waits for before other streams read the map or its
+    // memory is used again.  Every wave releases its own stores first.
+    __threadfence();
+    __syncthreads();
     if (tid == 0) {
         DevStatus v = new_status(s_bad[0], s_bad[1]);
         for (int t = 0; t < kTiles; ++t) v.key_mismatch |= s_mis[t];
@@ -360,7 +366,6 @@ __global__ __launch_bounds__(kThreads) void k_inv_small(
         counts->identity = v.key_mismatch == 0 ? 1 : 0;
         publish(v, st, pub);
     }
-    for (int k = tid; k < nk; k += kThreads) inv[k] = s_inv[k];
 }
 
 }  // namespace

@@ -124,3 +124,30 @@ def test_small_identity_inverse() -> None:
     for n, keys in ((1, 1), (4096, 4097), (10_000, 16_384)):
         bp = capi.inv_plan(_t(np.arange(n)), keys, None, 0)
         assert not bp.plan.inv and bp.plan.collisions == 0
+
+
+@pytest.mark.parametrize("wait", [True, False])
+@pytest.mark.parametrize("n", [100, 4096, 16384])
+def test_inverse_map_is_stored_when_the_build_returns(n: int, wait: bool) -> None:
+    """Once the build (or the validation of one that did not wait) has returned, another stream may read the
+    map: a copy that waits for nothing else, into memory that still holds the previous map before the build."""
+
+    from relmo_amd import capi
+
+    side = torch.cuda.Stream()
+    rng = np.random.default_rng(n)
+    for _ in range(20):
+        keys = rng.permutation(n)
+        kt = _t(keys)
+        torch.cuda.synchronize()
+        bp = capi.inv_plan(kt, n, None, 0, wait=wait, snapshot=True)
+        if not wait:
+            capi.validate(bp)
+        with torch.cuda.stream(side):
+            got = bp.inv.clone()
+            snap = bp._i32(bp.plan.snap_keys, n).clone()
+        side.synchronize()
+        assert np.array_equal(_np(got), np.argsort(keys))
+        plain = _arr(bp, "snap_key_plain", -(-n // 4096))
+        assert np.array_equal(np.where(np.repeat(plain, 4096)[:n] != 0, np.arange(n), _np(snap)), keys)
+
