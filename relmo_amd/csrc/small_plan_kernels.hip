@@ -76,7 +76,8 @@ __device__ __forceinline__ uint32_t key_word(uint32_t deg) {
 // into one word each (one pass of up to 7 bits, or two), offsets from a running
 // maximum of the segments' ends, then the per-key index.  Bound by latency: some
 // 15 barriers and, per sort pass and 64 edges of a wave, about a hundred
-// instructions of ranking.  Wave w owns positions [w * per, w * per + per) in
+// instructions of ranking.  keys and gathers are read before the validation is
+// published and not after it.  Wave w owns positions [w * per, w * per + per) in
 // rounds of 64, so the order (wave, round, lane) is the edge order.
 template <int ITEMS>
 __global__ __launch_bounds__(kThreads) void k_csr_small(
@@ -273,24 +274,23 @@ __global__ __launch_bounds__(kThreads) void k_csr_small(
     }
     __syncthreads();
 
-    // ---- the gathered rows in key order, and without the hubs' segments
+    // ---- the gathered rows in key order, and without the hubs' segments: from
+    // the snapshot, for the caller may change its arrays once the validation is
+    // published
     const bool any_hub = (total >> kHubShift) != 0u;
 #pragma unroll 1
     for (int q = tid; q < n; q += 4 * kThreads) {
-        uint32_t it[4];
-        int64_t g[4];
+        uint32_t it[4], g[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             it[j] = sk[min(q + j * kThreads, n - 1)];
-            g[j] = gathers != nullptr ? gathers[it[j] & kPosMask] : 0;
+            g[j] = gathers != nullptr ? a.snap_gathers[it[j] & kPosMask] : it[j] & kPosMask;
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int p = q + j * kThreads;
             if (p >= n) continue;
-            uint32_t bad = 0;
-            const int32_t v = static_cast<int32_t>(
-                gathers != nullptr ? narrow(g[j], gather_bound, 0, bad) : it[j] & kPosMask);
+            const int32_t v = static_cast<int32_t>(g[j]);
             a.gather_sorted[p] = v;
             if (any_hub) {
                 const uint32_t x = sx[it[j] >> kPosBits];

@@ -151,3 +151,30 @@ def test_inverse_map_is_stored_when_the_build_returns(n: int, wait: bool) -> Non
         plain = _arr(bp, "snap_key_plain", -(-n // 4096))
         assert np.array_equal(np.where(np.repeat(plain, 4096)[:n] != 0, np.arange(n), _np(snap)), keys)
 
+
+
+@pytest.mark.parametrize("num_keys,num_edges", [(50, 4096), (16384, 16384)])
+def test_csr_build_reads_no_index_array_after_it_returns(num_keys: int, num_edges: int) -> None:
+    """A build that returns once the indices are validated leaves them to the caller: overwritten on another
+    stream that waits for nothing, they change neither the sorted rows nor the snapshot."""
+
+    from relmo_amd import capi
+
+    side = torch.cuda.Stream()
+    rng = np.random.default_rng(num_keys)
+    for _ in range(20):
+        keys, gathers = rng.integers(0, num_keys, num_edges), rng.permutation(num_edges)
+        kt, gt = _t(keys), _t(gathers)
+        torch.cuda.synchronize()
+        bp = capi.csr_plan(kt, num_keys, gt, num_edges, wait_counts=False)
+        with torch.cuda.stream(side):
+            gt.fill_(-1)
+            kt.fill_(-1)
+        torch.cuda.synchronize()
+        capi.read_counts(bp, kt)
+        offsets, perm = oracle.csr_build(keys, num_keys)
+        assert np.array_equal(_np(bp.offsets), offsets)
+        assert np.array_equal(_np(bp.gather_sorted), gathers[perm])
+        short = np.repeat(np.diff(offsets) <= bp.plan.hub_threshold, np.diff(offsets))
+        assert np.array_equal(_np(bp.short_gather), gathers[perm][short])
+        assert capi.plan_match(_t(keys), _t(gathers), [bp]) == [True]
