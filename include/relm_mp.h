@@ -475,6 +475,7 @@ int relm_mp_pack_index(const relm_mp_index_part* parts, int32_t num_parts, int64
  * row-major) form range k and share row k of gamma, beta and add [num_ranges,
  * width] (add may be NULL: zero):
  *   y[r] = mish(beta[k] + gamma[k] * (s[r] + add[k])),  mish(u) = u tanh(softplus(u)).
+ * y may equal s (the same buffer; no other overlap).
  * range_start: num_ranges + 1 ascending host values from 0 to rows,
  * 1 <= num_ranges <= RELM_MP_FILM_MAX_RANGES. */
 #define RELM_MP_FILM_MAX_RANGES 16
@@ -493,7 +494,8 @@ int64_t relm_mp_film_mish_blocks(const int64_t* range_start, int32_t num_ranges)
  * row order) the column sums of du * (s + add[k]) and of du over its rows, each
  * fp32 term added in fp64: summed over range k's blocks they are the gradients of
  * gamma[k] and of beta[k] (that of add[k] is gamma[k] times the latter).
- * partial_blocks >= relm_mp_film_mish_blocks(...). */
+ * partial_blocks >= relm_mp_film_mish_blocks(...).  ds may equal s or dy (the same
+ * buffer; no other overlap). */
 int relm_mp_film_mish_backward(const float* s, const float* dy, int64_t rows, int64_t width,
                                const int64_t* range_start, int32_t num_ranges, const float* gamma,
                                const float* beta, const float* add, float* ds, double* partial,
@@ -501,7 +503,8 @@ int relm_mp_film_mish_backward(const float* s, const float* dy, int64_t rows, in
 
 /* relm_mp_film_mish_backward with the block sums added up on the device: sums
  * [num_ranges, 2, width] (float32) receives per range the gradients of gamma[k] and
- * of beta[k] (zero for an empty range), added in fp64 and rounded once.  workspace:
+ * of beta[k] (zero for an empty range), added in fp64 and rounded once.  ds may equal
+ * s or dy.  workspace:
  * relm_mp_film_mish_backward_sums_workspace_size(...) bytes, 8-byte aligned. */
 size_t relm_mp_film_mish_backward_sums_workspace_size(const int64_t* range_start, int32_t num_ranges,
                                                       int64_t width);

@@ -322,12 +322,19 @@ int64_t film_rows_per_block(const FilmLayout& L, int64_t rows, int least, int mo
     return static_cast<int64_t>(per_thread) * L.phases;
 }
 
-// 4 floats to a unit, at any alignment; rows narrower than that go one by one.
-int film_vec(int64_t width) { return width >= 4 ? 4 : 1; }
+// 4 floats to a unit, at any alignment; rows narrower than that go one by one,
+// and so do rows whose last unit would share columns with the one before it
+// where the output takes the place of an input: a column must not be read again
+// after another thread has written it.
+int film_vec(int64_t width, bool in_place = false) {
+    return width >= 4 && !(in_place && width % 4 != 0) ? 4 : 1;
+}
 
 hipError_t film_backward(const float* s, const float* dy, int64_t width, const FilmRanges& R,
-                         const FilmLayout& L, int V, const float* gamma, const float* beta,
-                         const float* add, float* ds, double* partial, hipStream_t st) {
+                         const float* gamma, const float* beta, const float* add, float* ds,
+                         double* partial, hipStream_t st) {
+    const int V = film_vec(width, ds == s || ds == dy);
+    const FilmLayout L = film_layout(width, V);
     const dim3 grid(static_cast<unsigned>(R.first_block[kMaxRanges] * L.chunks));
     const size_t lds = static_cast<size_t>(L.phases) * L.units * V * 2 * sizeof(double);
     const auto kernel = V == 4 ? k_film_mish_backward<4> : k_film_mish_backward<1>;
@@ -348,7 +355,7 @@ hipError_t launch_film_mish(const float* s, int64_t width, const int64_t* range_
                             const float* add, float* y, hipStream_t st) {
     const int64_t rows = range_start[num_ranges];
     if (rows == 0 || width == 0) return hipSuccess;
-    const int V = film_vec(width);
+    const int V = film_vec(width, y == s);
     const FilmLayout L = film_layout(width, V);
     const FilmRanges R = film_ranges(range_start, num_ranges, film_rows_per_block(L, rows, 4, 16));
     const dim3 grid(static_cast<unsigned>(R.first_block[kMaxRanges] * L.chunks));
@@ -362,9 +369,8 @@ hipError_t launch_film_mish_backward(const float* s, const float* dy, int64_t wi
                                      const float* gamma, const float* beta, const float* add,
                                      float* ds, double* partial, hipStream_t st) {
     if (range_start[num_ranges] == 0 || width == 0) return hipSuccess;
-    const int V = film_vec(width);
     const FilmRanges R = film_ranges(range_start, num_ranges, RELM_MP_FILM_ROWS_PER_BLOCK);
-    return film_backward(s, dy, width, R, film_layout(width, V), V, gamma, beta, add, ds, partial, st);
+    return film_backward(s, dy, width, R, gamma, beta, add, ds, partial, st);
 }
 
 size_t film_sums_workspace(const int64_t* range_start, int32_t num_ranges, int64_t width) {
@@ -379,10 +385,9 @@ hipError_t launch_film_mish_backward_sums(const float* s, const float* dy, int64
                                           float* ds, float* sums, double* partial, hipStream_t st) {
     if (width == 0) return hipSuccess;
     const int64_t rows = range_start[num_ranges];
-    const int V = film_vec(width);
     const FilmRanges R = film_ranges(range_start, num_ranges, film_backward_rows(width, rows));
     if (rows > 0) {
-        const hipError_t e = film_backward(s, dy, width, R, film_layout(width, V), V, gamma, beta, add, ds, partial, st);
+        const hipError_t e = film_backward(s, dy, width, R, gamma, beta, add, ds, partial, st);
         if (e != hipSuccess) return e;
     }
     const int64_t cols = 2 * width;

@@ -161,6 +161,46 @@ def test_film_mish_backward_sums(width, starts) -> None:
         b0 += nb
 
 
+@pytest.mark.parametrize("width", [5, 131, 257, 400])  # the last unit shared, over chunks too, and not
+def test_film_mish_in_place(width: int) -> None:
+    """The output over the input (y over s, ds over s or dy): the bits of a call with buffers of its own."""
+
+    from relmo_amd import capi
+
+    g = torch.Generator(device=DEV).manual_seed(width)
+    rows, starts = 3001, [0, 1200, 3001]
+    s, dy = (torch.randn(rows, width, device=DEV, generator=g) for _ in range(2))
+    tables = [torch.randn(2, width, device=DEV, generator=g) for _ in range(3)]
+    ptrs = [capi._ptr(t) for t in tables]
+    arr, k = capi._starts(starts)
+    y = s.clone()
+    capi.check(capi.lib().relm_mp_film_mish(capi._ptr(y), rows, width, arr, k, *ptrs, capi._ptr(y), capi._stream(s)))
+    assert torch.equal(y, capi.film_mish(s, starts, *tables))
+    ds, partial = capi.film_mish_backward(dy, s, starts, *tables)
+    _, sums = capi.film_mish_backward_sums(dy, s, starts, *tables)
+    for over_s in (True, False):
+        for fold in (True, False):
+            a, d = s.clone(), dy.clone()
+            out = a if over_s else d
+            if fold:
+                got = torch.empty_like(sums)
+                n = capi.lib().relm_mp_film_mish_backward_sums_workspace_size(arr, k, width)
+                ws = torch.empty(n, dtype=torch.uint8, device=DEV)
+                capi.check(capi.lib().relm_mp_film_mish_backward_sums(
+                    capi._ptr(a), capi._ptr(d), rows, width, arr, k, *ptrs, capi._ptr(out), capi._ptr(got),
+                    capi._ptr(ws), n, capi._stream(s)))
+                # fp32 terms added in fp64 in another order, rounded to fp32 once
+                torch.testing.assert_close(got, sums, rtol=1.2e-7, atol=0)
+            else:
+                got = torch.empty_like(partial)
+                capi.check(capi.lib().relm_mp_film_mish_backward(
+                    capi._ptr(a), capi._ptr(d), rows, width, arr, k, *ptrs, capi._ptr(out), capi._ptr(got),
+                    partial.size(0), capi._stream(s)))
+                # 512 fp32 terms of a block in another order: at most 512 fp64 roundings of sums below 512 * max |term|
+                torch.testing.assert_close(got, partial, rtol=0, atol=512 * 512 * 2.3e-16 * 100)
+            assert torch.equal(out, ds)
+
+
 def test_film_mish_extremes_and_errors() -> None:
     """Large and very negative pre-activations (Mish is u and 0 there), and
     ranges that do not cover the rows."""
