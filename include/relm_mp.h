@@ -300,7 +300,8 @@ int relm_mp_plan_segment_reduce(int dtype, const relm_mp_plan* plan, const int64
                                 const void* table, int64_t emb, int64_t mode, void* out,
                                 void* scratch, size_t scratch_bytes, relm_mp_stream_t stream);
 /* grad_rel[num_keys, emb] = per key r, sum over its edges of
- * grad_out[d] * exp(rel_flat[r] - out[d]) with d the gathered row. */
+ * grad_out[d] * exp(rel_flat[r] - out[d]) with d the gathered row.  grad_rel may
+ * equal rel_flat, but not with a CSR plan that has hubs (their rows are written twice). */
 int relm_mp_plan_logsumexp_backward(int dtype, const relm_mp_plan* plan, const int64_t* gathers,
                                     const void* grad_out, const void* out, const void* rel_flat,
                                     int64_t emb, void* grad_rel, void* scratch,

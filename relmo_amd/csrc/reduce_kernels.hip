@@ -1329,10 +1329,13 @@ inline Geometry lanes_geometry(int64_t D, int V) {
     return {V, G, (vcols + G - 1) / G};
 }
 
+// One element also where the output takes the place of an input row by row and
+// lanes would share columns (lane_column): a column must not be read again after
+// another lane, past one slice another workgroup, has written it.
 template <typename T>
-Geometry choose_geometry(int64_t D) {
+Geometry choose_geometry(int64_t D, bool in_place = false) {
     constexpr int kVecMax = 16 / static_cast<int>(sizeof(T));
-    return lanes_geometry(D, D >= kVecMax ? kVecMax : 1);
+    return lanes_geometry(D, D >= kVecMax && !(in_place && D % kVecMax != 0) ? kVecMax : 1);
 }
 
 template <typename T, typename F>
@@ -1626,7 +1629,7 @@ int lse_backward_t(const relm_mp_plan& plan, const int64_t* gathers, const void*
             return hip_error(hipGetLastError(), "relm_mp logsumexp backward kernel");
         });
     }
-    const Geometry geo = choose_geometry<T>(emb);
+    const Geometry geo = choose_geometry<T>(emb, grad_rel == rel);
     return with_geometry<T>(geo, [&](auto vt, auto gt) -> int {
         constexpr int V = decltype(vt)::value;
         constexpr int G = decltype(gt)::value;
@@ -1739,14 +1742,7 @@ int rows_scale_t(const void* in_v, const int64_t* gather, int div_kind, const in
     const T* in = static_cast<const T*>(in_v);
     const T* base = static_cast<const T*>(base_v);
     T* out = static_cast<T*>(out_v);
-    Geometry geo = choose_geometry<T>(emb);
-    // in place, a column must not be read again after a second lane has written
-    // it: one element per lane where the lanes would share columns
-    if ((out == in || out == base) && emb % geo.V != 0) {
-        geo.V = 1;
-        geo.G = 64;
-        geo.slices = (emb + 63) / 64;
-    }
+    const Geometry geo = choose_geometry<T>(emb, out == in || out == base);
     return with_geometry<T>(geo, [&](auto vt, auto gt) -> int {
         constexpr int V = decltype(vt)::value;
         constexpr int G = decltype(gt)::value;

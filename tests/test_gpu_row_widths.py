@@ -5,6 +5,7 @@ gathers and the logsumexp backward), against torch in float64."""
 
 from __future__ import annotations
 
+import ctypes
 import math
 import os
 
@@ -98,3 +99,29 @@ def test_rows_scale_in_place_at_odd_width() -> None:
         capi.check(capi.lib().relm_mp_rows_scale(0, capi._ptr(x), None, capi.DIV_NONE, None, None, capi._ptr(out),
                                                  200, emb, capi._ptr(out), capi._stream(x)))
         assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("dtype,widths", [(torch.float32, (8, 33, 258, 515, 16387)), (torch.float64, (33, 131, 259))])
+def test_logsumexp_backward_in_place(dtype, widths) -> None:
+    """grad_rel over rel_flat, rows of several column slices among them: the bits of a call with a buffer of its
+    own, by the CSR plan of a flat_src that repeats (without hubs) and by the inverse plan of one that does not."""
+
+    from relmo_amd import capi
+
+    g = torch.Generator(device=DEV).manual_seed(3)
+    rows, keys = 900, 40
+    for emb in widths:
+        rel = torch.randn(rows, emb, device=DEV, dtype=dtype, generator=g)
+        grad, out = (torch.randn(keys, emb, device=DEV, dtype=dtype, generator=g) for _ in range(2))
+        for repeats in (True, False):
+            flat = torch.randint(0, rows, (4000,), device=DEV, generator=g) if repeats else torch.randperm(rows, device=DEV, generator=g)
+            dst = torch.randint(0, keys, (flat.numel(),), device=DEV, generator=g)
+            bp = capi.csr_plan(flat, rows, dst, keys) if repeats else capi.inv_plan(flat, rows, dst, keys)
+            want = capi.plan_logsumexp_backward(bp, grad, out, rel, None if repeats else dst)
+            over = rel.clone()
+            n = capi.lib().relm_mp_plan_compute_scratch_bytes(ctypes.byref(bp.plan), emb, capi._dtype(rel), 1)
+            ws = torch.empty(max(n, 1), dtype=torch.uint8, device=DEV)
+            capi.check(capi.lib().relm_mp_plan_logsumexp_backward(
+                capi._dtype(rel), ctypes.byref(bp.plan), None if repeats else capi._ptr(dst), capi._ptr(grad), capi._ptr(out),
+                capi._ptr(over), emb, capi._ptr(over), capi._ptr(ws), ws.numel(), capi._stream(rel)))
+            assert torch.equal(over, want), (emb, repeats)
