@@ -51,15 +51,16 @@ __device__ __forceinline__ unsigned long long match_digit(uint32_t digit,
 }
 
 // V elements of a row as one load / store, at any address aligned to one
-// element: global memory takes 8- and 16-byte accesses at dword alignment, so
-// rows of any width and column offset move in the widest pieces.
+// element: global memory takes 8- and 16-byte accesses at dword alignment.  The
+// elements are spelled out one by one and the compiler joins them: written as
+// one vector access of a type of lower alignment, the kernels got other
+// schedules and registers, and rows of whole lanes were slower (sum of 16.8 M
+// gathered rows of 64 floats 739 against 757 us, the gather of 4.2 M of 128
+// floats 603 against 618, the divided sum's walker 96 VGPRs against 110).
 template <typename T, int V>
 struct alignas(sizeof(T) * V) Pack {  // of a value in registers or LDS
     T v[V];
 };
-
-template <typename T, int V>
-using PackVec = T __attribute__((ext_vector_type(V), aligned(sizeof(T))));
 
 template <typename T, int V>
 __device__ __forceinline__ Pack<T, V> pack_fill(T x) {
@@ -70,41 +71,33 @@ __device__ __forceinline__ Pack<T, V> pack_fill(T x) {
 }
 
 template <typename T, int V>
-__device__ __forceinline__ Pack<T, V> pack_of(PackVec<T, V> x) {
+__device__ __forceinline__ Pack<T, V> pack_load(const T* ptr) {
     Pack<T, V> p;
 #pragma unroll
-    for (int i = 0; i < V; ++i) p.v[i] = x[i];
+    for (int i = 0; i < V; ++i) p.v[i] = ptr[i];
     return p;
 }
 
 template <typename T, int V>
-__device__ __forceinline__ PackVec<T, V> pack_vec(const Pack<T, V>& p) {
-    PackVec<T, V> x;
-#pragma unroll
-    for (int i = 0; i < V; ++i) x[i] = p.v[i];
-    return x;
-}
-
-template <typename T, int V>
-__device__ __forceinline__ Pack<T, V> pack_load(const T* ptr) {
-    return pack_of<T, V>(*reinterpret_cast<const PackVec<T, V>*>(ptr));
-}
-
-template <typename T, int V>
 __device__ __forceinline__ void pack_store(T* ptr, const Pack<T, V>& p) {
-    *reinterpret_cast<PackVec<T, V>*>(ptr) = pack_vec(p);
+#pragma unroll
+    for (int i = 0; i < V; ++i) ptr[i] = p.v[i];
 }
 
 // Streaming load: rows read once, kept out of the way of reused rows in L2.
 template <typename T, int V>
 __device__ __forceinline__ Pack<T, V> pack_load_stream(const T* ptr) {
-    return pack_of<T, V>(__builtin_nontemporal_load(reinterpret_cast<const PackVec<T, V>*>(ptr)));
+    Pack<T, V> p;
+#pragma unroll
+    for (int i = 0; i < V; ++i) p.v[i] = __builtin_nontemporal_load(ptr + i);
+    return p;
 }
 
 // Streaming store: the written rows are not re-read by this kernel.
 template <typename T, int V>
 __device__ __forceinline__ void pack_store_stream(T* ptr, const Pack<T, V>& p) {
-    __builtin_nontemporal_store(pack_vec(p), reinterpret_cast<PackVec<T, V>*>(ptr));
+#pragma unroll
+    for (int i = 0; i < V; ++i) __builtin_nontemporal_store(p.v[i], ptr + i);
 }
 
 // Maximum that propagates NaN like ATen's amax (a NaN operand wins).

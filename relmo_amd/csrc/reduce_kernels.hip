@@ -176,8 +176,9 @@ struct SumOp {
     using Partial = SumPartial<T, V>;
     const T* __restrict__ table;
     int64_t D;
-    uint32_t col;  // first column of the lane; 0 past the row (the values are not used)
-    bool colok;   // the lane has columns
+    int64_t col;   // first column of the lane
+    bool colok;    // the lane has columns
+    int64_t lcol;  // column the lane loads: col, or 0 past the row (value unused)
     Pack<T, V> x[U];
     Pack<T, V> acc;
     Rows rows;  // layout of the table rows
@@ -198,7 +199,7 @@ struct SumOp {
     // accumulated, lanes past the row never stored.
     __device__ __forceinline__ void load(const int32_t (&idx)[U], int) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) x[u] = pack_load<T, V>(table + rows(idx[u], D) + col);
+        for (int u = 0; u < U; ++u) x[u] = pack_load<T, V>(table + rows(idx[u], D) + lcol);
     }
     // Rows u >= cnt (or !valid) leave the accumulator as it is: selects, not
     // branches, so the loads stay unconditional.
@@ -257,8 +258,9 @@ struct LseOp {
     using Partial = LsePartial<T, V>;
     const T* __restrict__ table;
     int64_t D;
-    uint32_t col;
+    int64_t col;
     bool colok;
+    int64_t lcol;  // as SumOp::lcol
     Pack<T, V> x[U];
     Pack<T, V> m, s;
 
@@ -285,7 +287,7 @@ struct LseOp {
     // as SumOp::load
     __device__ __forceinline__ void load(const int32_t (&idx)[U], int) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) x[u] = pack_load<T, V>(table + row_offset(idx[u], D) + col);
+        for (int u = 0; u < U; ++u) x[u] = pack_load<T, V>(table + row_offset(idx[u], D) + lcol);
     }
     // Batch maximum, then the rescaled sum; rows u >= cnt are masked by
     // selects (no branch, so the loads stay unconditional).  While the maximum
@@ -357,15 +359,16 @@ struct LseBwdOp {
     const T* __restrict__ out;
     const T* __restrict__ rel;
     int64_t D;
-    uint32_t col;
+    int64_t col;
     bool colok;
+    int64_t lcol;  // as SumOp::lcol
     Pack<T, V> g[U], o[U];
     Pack<T, V> xr, acc;
 
     // key is a valid rel row (hub chunks outside the plan pass row 0)
     __device__ __forceinline__ void begin(int64_t key, bool) {
         acc = pack_fill<T, V>(T(0));
-        xr = pack_load<T, V>(rel + key * D + col);
+        xr = pack_load<T, V>(rel + key * D + lcol);
     }
     __device__ __forceinline__ void restart(bool head, int64_t key) {
         if (head) begin(key, true);
@@ -374,7 +377,7 @@ struct LseBwdOp {
     __device__ __forceinline__ void load(const int32_t (&idx)[U], int) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const uint64_t off = row_offset(idx[u], D) + col;
+            const uint64_t off = row_offset(idx[u], D) + lcol;
             g[u] = pack_load<T, V>(grad_out + off);
             o[u] = pack_load<T, V>(out + off);
         }
@@ -401,24 +404,32 @@ struct LseBwdOp {
 // Minimum waves per SIMD asked of the compiler for the walker and the hub
 // chunks (HIP's second launch bound), which caps their VGPRs: the fp32 sum and
 // logsumexp over dense rows fit 96 VGPRs in the walker (5 waves instead of 4 at
-// 116), the sum of rows of more than 32 floats 80 (6 waves; narrower ones would
-// spill), and 80 in the hub chunks (6 instead of 5 at 93) without spilling; the
-// other ops (fp64, grouped rows, the logsumexp backward) would spill, and keep
-// the compiler's choice.
-template <class Op, int G>
+// 116) and 80 in the hub chunks (6 instead of 5 at 93) without spilling, the
+// logsumexp backward 128 in the walker but for two values (4 instead of 3 at
+// 148: 2 M rows of 32 floats with a message each 201 us, 186 with 4; 1 M rows with
+// 16 each 728 and 745); the other ops (fp64, grouped rows) would spill, and keep
+// the compiler's choice.  6 waves for the walker's sum of rows of more than 32
+// floats took 1,011 us on 16.8 M rows of 64 against 1,001 with 5, and spilled
+// with the scaling epilogue.
+template <class Op>
 struct WaveFloor {
     static constexpr int walk = 1;
     static constexpr int hub = 1;
 };
-template <int V, int U, int G>
-struct WaveFloor<SumOp<float, V, U, DenseRows>, G> {
-    static constexpr int walk = G >= 16 ? 6 : 5;
-    static constexpr int hub = 6;
-};
-template <int V, int U, int G>
-struct WaveFloor<LseOp<float, V, U>, G> {
+template <int V, int U>
+struct WaveFloor<SumOp<float, V, U, DenseRows>> {
     static constexpr int walk = 5;
     static constexpr int hub = 6;
+};
+template <int V, int U>
+struct WaveFloor<LseOp<float, V, U>> {
+    static constexpr int walk = 5;
+    static constexpr int hub = 6;
+};
+template <int V, int U>
+struct WaveFloor<LseBwdOp<float, V, U>> {
+    static constexpr int walk = 4;
+    static constexpr int hub = 1;
 };
 
 // Stores the result as is.
@@ -496,7 +507,7 @@ __global__ __launch_bounds__(kThreads) void k_fill(T* __restrict__ p, int64_t n,
 // whose label differs from the next one stores its key's result - no
 // per-key loop, so the row groups of a wave stay in step.
 template <typename T, int V, int G, class Op, class Epi>
-__global__ __launch_bounds__(kThreads, (WaveFloor<Op, G>::walk)) void k_walk_items(
+__global__ __launch_bounds__(kThreads, WaveFloor<Op>::walk) void k_walk_items(
     const int32_t* __restrict__ short_off, const int32_t* __restrict__ short_gather_in,
     const int32_t* __restrict__ gather_sorted, const int32_t* __restrict__ item_first,
     const int32_t* __restrict__ item_short, const relm_mp_plan_counts* __restrict__ pc,
@@ -520,9 +531,9 @@ __global__ __launch_bounds__(kThreads, (WaveFloor<Op, G>::walk)) void k_walk_ite
     __shared__ uint32_t s_scan[kThreads / kWave];
     const int gl = static_cast<int>(threadIdx.x) & (G - 1);
     const int grp = static_cast<int>(threadIdx.x) / G;
-    const uint32_t lane_col = lane_column<V, G>(gl, op.D);
-    op.colok = lane_col < op.D;
-    op.col = op.colok ? lane_col : 0;
+    op.col = lane_column<V, G>(gl, op.D);
+    op.colok = op.col < op.D;
+    op.lcol = op.colok ? op.col : 0;
     const int64_t D = op.D;
     const int64_t num_items = pc->num_items;
     const int64_t num_short = pc->num_short;
@@ -709,7 +720,7 @@ __device__ __forceinline__ int hub_slot(int p) { return p + (p >> 5); }
 // LDS with coalesced loads, row group g folds slice g of the chunk, the
 // slices are folded in order by group 0; a single-chunk hub is finished here.
 template <typename T, int V, int G, class Op, class Epi>
-__global__ __launch_bounds__(kThreads, (WaveFloor<Op, G>::hub)) void k_hub_chunks(
+__global__ __launch_bounds__(kThreads, WaveFloor<Op>::hub) void k_hub_chunks(
     const int32_t* __restrict__ offsets, const int32_t* __restrict__ gs, int64_t num_edges,
     const int32_t* __restrict__ hub_key, const int32_t* __restrict__ hub_chunk_base,
     const int32_t* __restrict__ chunk_hub, const relm_mp_plan_counts* __restrict__ pc,
@@ -722,9 +733,9 @@ __global__ __launch_bounds__(kThreads, (WaveFloor<Op, G>::hub)) void k_hub_chunk
     __shared__ int32_t s_gs[kChunkSize + kChunkSize / 32];
     const int gl = static_cast<int>(threadIdx.x) & (G - 1);
     const int grp = static_cast<int>(threadIdx.x) / G;
-    const uint32_t lane_col = lane_column<V, G>(gl, op.D);
-    op.colok = lane_col < op.D;
-    op.col = op.colok ? lane_col : 0;
+    op.col = lane_column<V, G>(gl, op.D);
+    op.colok = op.col < op.D;
+    op.lcol = op.colok ? op.col : 0;
     const int64_t D = op.D;
     const int64_t num_hubs = pc->num_hubs;
     const int64_t num_chunks = pc->num_chunks;
