@@ -1016,7 +1016,10 @@ __global__ __launch_bounds__(kThreads) void k_gather_inv(const int32_t* __restri
 // 16-byte piece at an odd place does not (each then costs two).  Backward of 4.2
 // M messages of 30 floats on 145,216 keys: 125 us by units, 151 by rows in 8-byte
 // lanes, 220 in 16-byte pieces across the seams; its logsumexp step 548, 560 and
-// 774 us.  A thread keeps UNITS units in flight, kThreads apart (4 and 16 were
+// 774 us.  Rows that fill a group's lanes, where a row's index is read once and not
+// once per unit, gain too: of rows in lanes of the same size, units take 0.97 at 31
+// and 62 floats, 0.97 to 1.04 at 63, 0.96 at 126, 0.65 at 127 and 0.73 at 254 (the
+// gather of 268 M floats), the logsumexp backward 0.98, 0.98, 0.98, 0.77 and 0.84.  A thread keeps UNITS units in flight, kThreads apart (4 and 16 were
 // up to 8% slower than 8 for the gather).
 constexpr int kGatherUnits = 8;
 constexpr int kLseUnits = 4;
@@ -1328,11 +1331,6 @@ struct Geometry {
     int64_t slices;
 };
 
-// 16 bytes per lane whatever the alignment (lane_column), one element where a
-// row has fewer.  Narrower lanes where the rows or the base are not aligned cost
-// the reductions more than the straddled lines do: 2 M argument slots of 128 floats at an
-// 8-byte aligned column 575 us in 8-byte lanes, 503 in 16-byte ones; the hub
-// chunks of 3 M messages of 33 floats 120 us in 4-byte lanes, 106 in 16-byte ones.
 inline Geometry lanes_geometry(int64_t D, int V) {
     const int64_t vcols = (D + V - 1) / V;
     int G = 4;
@@ -1340,16 +1338,96 @@ inline Geometry lanes_geometry(int64_t D, int V) {
     return {V, G, (vcols + G - 1) / G};
 }
 
-// One element also where the output takes the place of an input row by row and
-// lanes would share columns (lane_column): a column must not be read again after
+template <typename T>
+constexpr int kVecMax = 16 / static_cast<int>(sizeof(T));
+
+// Gathers and row scaling: 16 bytes per lane whatever the alignment
+// (lane_column), one element where a row has fewer.  2 M argument slots of 128
+// floats at an 8-byte aligned column 575 us in 8-byte lanes, 503 in 16-byte ones.
+// Where the output takes the place of an input row by row and lanes would share
+// columns, the widest lanes that do not: a column must not be read again after
 // another lane, past one slice another workgroup, has written it.
 template <typename T>
 Geometry choose_geometry(int64_t D, bool in_place = false) {
-    constexpr int kVecMax = 16 / static_cast<int>(sizeof(T));
-    return lanes_geometry(D, D >= kVecMax && !(in_place && D % kVecMax != 0) ? kVecMax : 1);
+    if (in_place && D % kVecMax<T> != 0) return lanes_geometry(D, D % 2 == 0 && kVecMax<T> > 2 ? 2 : 1);
+    return lanes_geometry(D, D >= kVecMax<T> ? kVecMax<T> : 1);
 }
 
-template <typename T, typename F>
+// Elements per lane of the CSR reductions.  Rows of whole 16-byte lanes that
+// start on 16 bytes take those.  In others such an access straddles lines, and
+// narrower lanes, each a whole access, are faster while one slice (a row group of
+// 64 lanes) holds the row and most of its lanes work.  The factors below are the
+// widest lanes' time over that of the narrower ones, walker: segments of 8 and of
+// 40 messages, hubs: of 4,000, over 67 M floats or 34 M doubles.
+enum class Reduction { kSum, kScaled, kDivided, kLse, kLseBackward };
+
+template <bool HUB_PAIRS>
+struct CsrLanes {
+    int walk;
+    int hub;
+    static constexpr bool kHubPairs = HUB_PAIRS;  // hub may be 2 floats
+};
+
+// Walker.  Floats: pairs (1.00 to 1.09 at even widths, where an access is whole;
+// shared ones at odd widths 0.98 to 1.07); single ones at odd widths of 17 to 31
+// but for the scaled sum (1.01 to 1.10; pairs 1.00 to 1.05) and of 49 to 63 without
+// an epilogue (1.01 to 1.09; pairs 1.00 to 1.03).  16 bytes where rows are short (below 16: 0.93 to 1.05) or
+// would take further slices (130 to 254: 0.70 to 0.95; sums of 258 and more 0.89 to
+// 1.00, the other ops 0.89 to 1.00 where the slices halve and up to 1.11 where three
+// become two), and for the sums with an epilogue where pairs would leave a third of
+// the group idle (33 to 38, 65 to 79: 0.87 to 1.02, next to 1.04 at 46 and 62).
+// Doubles: pairs where they halve the slices (65 to 127: 0.70 to 0.91; elsewhere
+// 0.94 to 1.12, 1.38 for the logsumexp of 3), and for the logsumexp of 33 to 63
+// (0.89 to 1.00).
+template <typename T>
+int walk_lanes(int64_t D, Reduction r) {
+    const auto slices = [D](int V) { return lanes_geometry(D, V).slices; };
+    if constexpr (sizeof(T) == 8) {
+        return 2 * slices(2) <= slices(1) || (r == Reduction::kLse && D > 32 && D < 64) ? 2 : 1;
+    } else {
+        if (D < 16) return D >= 4 ? 4 : 1;
+        const bool sum = r == Reduction::kSum || r == Reduction::kScaled;
+        if (D > 128) return sum || 2 * slices(4) <= slices(D % 2 == 0 ? 2 : 1) ? 4 : 2;
+        const bool epilogue = r == Reduction::kScaled || r == Reduction::kDivided;
+        if (epilogue && D > 32 && 3 * ((D + 1) / 2) <= 2 * lanes_geometry(D, 2).G) return 4;
+        const bool single = D < 32 ? r != Reduction::kScaled : D > 48 && D < 64 && !epilogue;
+        return D % 2 != 0 && single ? 1 : 2;
+    }
+}
+
+// Hub chunks.  Sums: the widest lanes (rows from the caches 0.61 to 1.02, from
+// memory 0.69 to 1.02 and up to 1.11 at 63 and 126 floats, which over 268 M are 0.97
+// and 1.01).  The logsumexp and its backward hold twice the values and merge them
+// across the groups: by widest lanes in groups of 64 the logsumexp takes 1.10 to
+// 1.54 and its backward up to 1.43, so rows that would need such groups go by the
+// widest lanes that divide them, as do the shortest (logsumexp below 16 floats 1.02
+// to 1.05, below 20 doubles 0.98 to 1.08; backward of 3 doubles 1.20).  In between
+// the widest lanes for the backward (0.64 to 0.96) and the logsumexp of more than 64
+// floats (0.81 to 0.93), else pairs (16-byte lanes 1.00 to 1.06).
+template <typename T>
+int hub_lanes(int64_t D, Reduction r) {
+    constexpr int W = kVecMax<T>;
+    const bool backward = r == Reduction::kLseBackward;
+    if (!backward && r != Reduction::kLse) return D >= W ? W : 1;
+    const int whole = W > 2 && D % 2 == 0 ? 2 : 1;
+    if (D > 32 * W) return whole;
+    if constexpr (sizeof(T) == 8) return D < (backward ? 5 : 20) ? 1 : 2;
+    if (D < 16) return backward && D >= 4 ? 2 : whole;
+    return backward || D > 64 ? W : 2;
+}
+
+// `aligned`: every row of the tables starts on 16 bytes.
+template <typename T, Reduction R>
+auto csr_lanes(int64_t D, bool aligned) {
+    using Lanes = CsrLanes<R == Reduction::kLse || R == Reduction::kLseBackward>;
+    if (aligned && D % kVecMax<T> == 0) return Lanes{kVecMax<T>, kVecMax<T>};
+    return Lanes{walk_lanes<T>(D, R), hub_lanes<T>(D, R)};
+}
+
+inline bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
+
+// Calls f(V, G) for a geometry; PAIRS: two floats to a lane are among its choices.
+template <typename T, bool PAIRS, typename F>
 int with_geometry(const Geometry& geo, F&& f) {
     auto by_g = [&](auto vt) -> int {
         switch (geo.G) {
@@ -1362,8 +1440,10 @@ int with_geometry(const Geometry& geo, F&& f) {
         }
         return set_error(RELM_MP_ERR_INVALID_ARGUMENT, "relm_mp: unsupported row geometry");
     };
-    constexpr int kVecMax = 16 / static_cast<int>(sizeof(T));
-    if (geo.V == kVecMax) return by_g(std::integral_constant<int, kVecMax>{});
+    if (geo.V == kVecMax<T>) return by_g(std::integral_constant<int, kVecMax<T>>{});
+    if constexpr (PAIRS && kVecMax<T> > 2) {
+        if (geo.V == 2) return by_g(std::integral_constant<int, 2>{});
+    }
     return by_g(std::integral_constant<int, 1>{});
 }
 
@@ -1380,9 +1460,8 @@ dim3 row_grid(int64_t rows, int G, int64_t slices, int rows_per_group = 1) {
 // for the units' division.
 template <typename T>
 int unit_width(int64_t D, int64_t num_edges, int64_t num_gather) {
-    constexpr int kVecMax = 16 / static_cast<int>(sizeof(T));
-    if (D % kVecMax == 0 || num_edges <= 0 || num_gather <= 0) return 0;
-    const int V = kVecMax > 2 && D > 2 && D % 2 == 0 ? 2 : 1;
+    if (D % kVecMax<T> == 0 || num_edges <= 0 || num_gather <= 0) return 0;
+    const int V = kVecMax<T> > 2 && D > 2 && D % 2 == 0 ? 2 : 1;
     return D / V > 1 && D / V <= kUnitsMaxRow ? V : 0;
 }
 
@@ -1444,42 +1523,57 @@ dim3 persistent_grid(const void* kernel, int64_t work, int64_t per_block, int64_
     return dim3(static_cast<unsigned>(bx), static_cast<unsigned>(slices));
 }
 
-// Runs the CSR reduction of `op` (items, hub chunks, hub combines) into out.
+// Runs a CSR reduction (items, hub chunks, hub combines) into out; make(vt, ut)
+// gives the op for V = vt and U = ut.
 // The item, hub and chunk counts are read from plan.counts on the device:
 // grids are sized by the host-side counts where the plan has them (>= 0),
 // else by the plan's capacities, and capped (persistent_grid).
-template <typename T, int V, int G, class Op, class Epi = NoEpilogue>
-int run_csr(const relm_mp_plan& plan, const Op& op, int64_t slices, T* partial, T* out,
-            hipStream_t s, const Epi& epi = Epi{}) {
-    using Partial = typename Op::Partial;
+template <typename T, class Lanes, class Make, class Epi = NoEpilogue>
+int run_csr(const relm_mp_plan& plan, const Lanes& lanes, int64_t emb, T* partial, T* out,
+            hipStream_t s, const Make& make, const Epi& epi = Epi{}) {
     if (plan.counts == nullptr)
         return set_error(RELM_MP_ERR_INVALID_ARGUMENT, "relm_mp: CSR plan without counts");
     const int64_t E = plan.num_edges;
     const int64_t items = plan.num_items >= 0 ? plan.num_items : item_capacity_for(plan.num_keys);
-    const void* walk = reinterpret_cast<const void*>(&k_walk_items<T, V, G, Op, Epi>);
-    hipLaunchKernelGGL((k_walk_items<T, V, G, Op, Epi>),
-                       persistent_grid(walk, items, kThreads / G, slices, 4), dim3(kThreads), 0, s,
-                       plan.short_off, plan.short_gather, plan.gather_sorted, plan.item_first,
-                       plan.item_short, plan.counts, plan.num_keys, out, op, epi);
-    int rc = hip_error(hipGetLastError(), "relm_mp item kernel");
+    const Geometry walk_geo = lanes_geometry(emb, lanes.walk);
+    const int rc = with_geometry<T, true>(walk_geo, [&](auto vt, auto gt) -> int {
+        constexpr int V = decltype(vt)::value;
+        constexpr int G = decltype(gt)::value;
+        const auto op = make(vt, std::integral_constant<int, batch_rows<G>()>{});
+        using Op = std::remove_const_t<decltype(op)>;
+        const void* walk = reinterpret_cast<const void*>(&k_walk_items<T, V, G, Op, Epi>);
+        hipLaunchKernelGGL((k_walk_items<T, V, G, Op, Epi>),
+                           persistent_grid(walk, items, kThreads / G, walk_geo.slices, 4), dim3(kThreads), 0, s,
+                           plan.short_off, plan.short_gather, plan.gather_sorted, plan.item_first,
+                           plan.item_short, plan.counts, plan.num_keys, out, op, epi);
+        return hip_error(hipGetLastError(), "relm_mp item kernel");
+    });
     // no hub when the counts say so, or when no segment can be longer than the threshold
     if (rc != RELM_MP_OK || plan.num_hubs == 0 || E <= kHubThreshold) return rc;
     const int64_t chunks = plan.num_chunks >= 0 ? plan.num_chunks : max_chunks(E);
-    const void* hub = reinterpret_cast<const void*>(&k_hub_chunks<T, V, G, Op, Epi>);
-    hipLaunchKernelGGL((k_hub_chunks<T, V, G, Op, Epi>), persistent_grid(hub, chunks, 1, slices, 8),
-                       dim3(kThreads), 0, s, plan.offsets, plan.gather_sorted, plan.num_edges,
-                       plan.hub_key, plan.hub_chunk_base, plan.chunk_hub, plan.counts, partial, out,
-                       op, epi);
-    rc = hip_error(hipGetLastError(), "relm_mp hub chunk kernel");
-    // no hub of more than one chunk when the counts say so, or when none fits
-    if (rc != RELM_MP_OK || plan.num_multi_hubs == 0 || E <= kChunkSize) return rc;
-    const int64_t multi = plan.num_multi_hubs >= 0 ? plan.num_multi_hubs : E / (kChunkSize + 1) + 1;
-    const void* comb = reinterpret_cast<const void*>(&k_hub_combine<T, V, G, Partial, Epi>);
-    hipLaunchKernelGGL((k_hub_combine<T, V, G, Partial, Epi>),
-                       persistent_grid(comb, multi, 1, slices, 8), dim3(kThreads), 0, s,
-                       op.D, plan.hub_key, plan.hub_chunk_base,
-                       plan.multi_hubs, plan.counts, static_cast<const T*>(partial), out, epi);
-    return hip_error(hipGetLastError(), "relm_mp hub combine kernel");
+    const Geometry hub_geo = lanes_geometry(emb, lanes.hub);
+    return with_geometry<T, Lanes::kHubPairs>(hub_geo, [&](auto vt, auto gt) -> int {
+        constexpr int V = decltype(vt)::value;
+        constexpr int G = decltype(gt)::value;
+        const auto op = make(vt, std::integral_constant<int, batch_rows<G>()>{});
+        using Op = std::remove_const_t<decltype(op)>;
+        using Partial = typename Op::Partial;
+        const void* hub = reinterpret_cast<const void*>(&k_hub_chunks<T, V, G, Op, Epi>);
+        hipLaunchKernelGGL((k_hub_chunks<T, V, G, Op, Epi>), persistent_grid(hub, chunks, 1, hub_geo.slices, 8),
+                           dim3(kThreads), 0, s, plan.offsets, plan.gather_sorted, plan.num_edges,
+                           plan.hub_key, plan.hub_chunk_base, plan.chunk_hub, plan.counts, partial, out,
+                           op, epi);
+        const int hrc = hip_error(hipGetLastError(), "relm_mp hub chunk kernel");
+        // no hub of more than one chunk when the counts say so, or when none fits
+        if (hrc != RELM_MP_OK || plan.num_multi_hubs == 0 || E <= kChunkSize) return hrc;
+        const int64_t multi = plan.num_multi_hubs >= 0 ? plan.num_multi_hubs : E / (kChunkSize + 1) + 1;
+        const void* comb = reinterpret_cast<const void*>(&k_hub_combine<T, V, G, Partial, Epi>);
+        hipLaunchKernelGGL((k_hub_combine<T, V, G, Partial, Epi>),
+                           persistent_grid(comb, multi, 1, hub_geo.slices, 8), dim3(kThreads), 0, s,
+                           emb, plan.hub_key, plan.hub_chunk_base,
+                           plan.multi_hubs, plan.counts, static_cast<const T*>(partial), out, epi);
+        return hip_error(hipGetLastError(), "relm_mp hub combine kernel");
+    });
 }
 
 // group > 0: the output rows are grouped (GroupedRows{group, group_stride}).
@@ -1516,17 +1610,10 @@ int gather_last_t(const relm_mp_plan& plan, const int64_t* gathers, const void* 
     if (group > 0) {
         const Geometry geo = choose_geometry<T>(emb);
         const GroupedRows rows{static_cast<uint32_t>(group), static_cast<uint64_t>(group_stride)};
-        return with_geometry<T>(
+        return with_geometry<T, false>(
             geo, [&](auto vt, auto gt) -> int { return launch(vt, gt, geo, rows); });
     }
     const int unit = plan.kind == RELM_MP_PLAN_INVERSE ? unit_width<T>(emb, plan.num_edges, plan.num_gather) : 0;
-    // Rows of an odd width that leave at most one lane in 32 idle (31, 63, 127
-    // floats): one element per lane, where a row's index is read once and not
-    // once per unit - 4 M rows of 31 366 us against 391, 2 M of 63 472 against 491.
-    const Geometry single = lanes_geometry(emb, 1);
-    if (unit == 1 && 32 * emb >= 31 * single.G * single.slices)
-        return with_geometry<T>(
-            single, [&](auto vt, auto gt) -> int { return launch(vt, gt, single, DenseRows{}); });
     if (unit > 0) {
         return with_unit<T>(unit, [&](auto vt) -> int {
             constexpr int V = decltype(vt)::value;
@@ -1543,7 +1630,7 @@ int gather_last_t(const relm_mp_plan& plan, const int64_t* gathers, const void* 
         });
     }
     const Geometry geo = choose_geometry<T>(emb);
-    return with_geometry<T>(geo,
+    return with_geometry<T, false>(geo,
                             [&](auto vt, auto gt) -> int { return launch(vt, gt, geo, DenseRows{}); });
 }
 
@@ -1555,17 +1642,15 @@ int segment_sum_grouped_t(const relm_mp_plan& plan, const void* table_v, int64_t
     const T* table = static_cast<const T*>(table_v);
     T* out = static_cast<T*>(out_v);
     T* partial = static_cast<T*>(scratch);
-    const Geometry geo = choose_geometry<T>(emb);
-    return with_geometry<T>(geo, [&](auto vt, auto gt) -> int {
-        constexpr int V = decltype(vt)::value;
-        constexpr int G = decltype(gt)::value;
-        constexpr int U = batch_rows<G>();
-        SumOp<T, V, U, GroupedRows> op{};
+    const auto make = [&](auto vt, auto ut) {
+        SumOp<T, decltype(vt)::value, decltype(ut)::value, GroupedRows> op{};
         op.table = table;
         op.D = emb;
         op.rows = GroupedRows{static_cast<uint32_t>(group), static_cast<uint64_t>(group_stride)};
-        return run_csr<T, V, G>(plan, op, geo.slices, partial, out, s);
-    });
+        return op;
+    };
+    const bool aligned = aligned16(table) && group_stride % kVecMax<T> == 0;
+    return run_csr<T>(plan, csr_lanes<T, Reduction::kSum>(emb, aligned), emb, partial, out, s, make);
 }
 
 template <typename T, int MODE>
@@ -1574,23 +1659,16 @@ int segment_reduce_t(const relm_mp_plan& plan, const void* table_v, int64_t emb,
     const T* table = static_cast<const T*>(table_v);
     T* out = static_cast<T*>(out_v);
     T* partial = static_cast<T*>(scratch);
-    const Geometry geo = choose_geometry<T>(emb);
-    return with_geometry<T>(geo, [&](auto vt, auto gt) -> int {
-        constexpr int V = decltype(vt)::value;
-        constexpr int G = decltype(gt)::value;
-        constexpr int U = batch_rows<G>();
-        if constexpr (MODE == RELM_MP_MODE_SUM) {
-            SumOp<T, V, U> op{};
-            op.table = table;
-            op.D = emb;
-            return run_csr<T, V, G>(plan, op, geo.slices, partial, out, s);
-        } else {
-            LseOp<T, V, U> op{};
-            op.table = table;
-            op.D = emb;
-            return run_csr<T, V, G>(plan, op, geo.slices, partial, out, s);
-        }
-    });
+    constexpr bool kLse = MODE == RELM_MP_MODE_LOGSUMEXP;
+    const auto make = [&](auto vt, auto ut) {
+        constexpr int V = decltype(vt)::value, U = decltype(ut)::value;
+        std::conditional_t<kLse, LseOp<T, V, U>, SumOp<T, V, U>> op{};
+        op.table = table;
+        op.D = emb;
+        return op;
+    };
+    constexpr Reduction kOp = kLse ? Reduction::kLse : Reduction::kSum;
+    return run_csr<T>(plan, csr_lanes<T, kOp>(emb, aligned16(table)), emb, partial, out, s, make);
 }
 
 template <typename T>
@@ -1601,17 +1679,14 @@ int segment_sum_scaled_t(const relm_mp_plan& plan, const void* table_v, int64_t 
     const T* base = static_cast<const T*>(base_v);
     T* out = static_cast<T*>(out_v);
     T* partial = static_cast<T*>(scratch);
-    const Geometry geo = choose_geometry<T>(emb);
-    return with_geometry<T>(geo, [&](auto vt, auto gt) -> int {
-        constexpr int V = decltype(vt)::value;
-        constexpr int G = decltype(gt)::value;
-        constexpr int U = batch_rows<G>();
-        SumOp<T, V, U> op{};
+    const auto make = [&](auto vt, auto ut) {
+        SumOp<T, decltype(vt)::value, decltype(ut)::value> op{};
         op.table = table;
         op.D = emb;
-        const ScaleEpilogue<T> epi{base, div_kind, plan.offsets, div_values};
-        return run_csr<T, V, G>(plan, op, geo.slices, partial, out, s, epi);
-    });
+        return op;
+    };
+    const ScaleEpilogue<T> epi{base, div_kind, plan.offsets, div_values};
+    return run_csr<T>(plan, csr_lanes<T, Reduction::kScaled>(emb, aligned16(table)), emb, partial, out, s, make, epi);
 }
 
 template <typename T>
@@ -1640,32 +1715,37 @@ int lse_backward_t(const relm_mp_plan& plan, const int64_t* gathers, const void*
             return hip_error(hipGetLastError(), "relm_mp logsumexp backward kernel");
         });
     }
+    if (plan.kind == RELM_MP_PLAN_CSR) {
+        const auto make = [&](auto vt, auto ut) {
+            LseBwdOp<T, decltype(vt)::value, decltype(ut)::value> op{};
+            op.grad_out = grad_out;
+            op.out = out;
+            op.rel = rel;
+            op.D = emb;
+            return op;
+        };
+        const bool aligned = aligned16(grad_out) && aligned16(out) && aligned16(rel);
+        auto lanes = csr_lanes<T, Reduction::kLseBackward>(emb, aligned);
+        if (grad_rel == rel) lanes.walk = choose_geometry<T>(emb, true).V;
+        return run_csr<T>(plan, lanes, emb, partial, grad_rel, s, make);
+    }
     const Geometry geo = choose_geometry<T>(emb, grad_rel == rel);
-    return with_geometry<T>(geo, [&](auto vt, auto gt) -> int {
+    return with_geometry<T, true>(geo, [&](auto vt, auto gt) -> int {
         constexpr int V = decltype(vt)::value;
         constexpr int G = decltype(gt)::value;
-        constexpr int U = batch_rows<G>();
-        if (plan.kind == RELM_MP_PLAN_INVERSE) {
-            const dim3 grid = row_grid(plan.num_keys, G, geo.slices, kLseRowsInFlight);
-            if (snap != nullptr) {
-                hipLaunchKernelGGL((k_lse_bwd_inv<T, V, G, GathersSnap>), grid, dim3(kThreads), 0, s,
-                                   plan.inv, plan.counts, plan.num_edges,
-                                   GathersSnap{snap->snap_keys, snap->snap_key_plain}, plan.num_gather,
-                                   grad_out, out, rel, plan.num_keys, emb, grad_rel, skip_on_collision);
-            } else {
-                hipLaunchKernelGGL((k_lse_bwd_inv<T, V, G, GathersI64>), grid, dim3(kThreads), 0, s,
-                                   plan.inv, plan.counts, plan.num_edges, GathersI64{gathers},
-                                   plan.num_gather, grad_out, out, rel, plan.num_keys, emb, grad_rel,
-                                   skip_on_collision);
-            }
-            return hip_error(hipGetLastError(), "relm_mp logsumexp backward kernel");
+        const dim3 grid = row_grid(plan.num_keys, G, geo.slices, kLseRowsInFlight);
+        if (snap != nullptr) {
+            hipLaunchKernelGGL((k_lse_bwd_inv<T, V, G, GathersSnap>), grid, dim3(kThreads), 0, s,
+                               plan.inv, plan.counts, plan.num_edges,
+                               GathersSnap{snap->snap_keys, snap->snap_key_plain}, plan.num_gather,
+                               grad_out, out, rel, plan.num_keys, emb, grad_rel, skip_on_collision);
+        } else {
+            hipLaunchKernelGGL((k_lse_bwd_inv<T, V, G, GathersI64>), grid, dim3(kThreads), 0, s,
+                               plan.inv, plan.counts, plan.num_edges, GathersI64{gathers},
+                               plan.num_gather, grad_out, out, rel, plan.num_keys, emb, grad_rel,
+                               skip_on_collision);
         }
-        LseBwdOp<T, V, U> op{};
-        op.grad_out = grad_out;
-        op.out = out;
-        op.rel = rel;
-        op.D = emb;
-        return run_csr<T, V, G>(plan, op, geo.slices, partial, grad_rel, s);
+        return hip_error(hipGetLastError(), "relm_mp logsumexp backward kernel");
     });
 }
 
@@ -1705,18 +1785,15 @@ int segment_sum_msgdiv_t(const relm_mp_plan& plan, const void* table_v, int64_t 
     const T* base = static_cast<const T*>(base_v);
     T* out = static_cast<T*>(out_v);
     T* partial = static_cast<T*>(scratch);
-    const Geometry geo = choose_geometry<T>(emb);
-    return with_geometry<T>(geo, [&](auto vt, auto gt) -> int {
-        constexpr int V = decltype(vt)::value;
-        constexpr int G = decltype(gt)::value;
-        constexpr int U = batch_rows<G>();
-        SumDivOp<T, V, U> op{};
+    const auto make = [&](auto vt, auto ut) {
+        SumDivOp<T, decltype(vt)::value, decltype(ut)::value> op{};
         op.table = table;
         op.D = emb;
         op.div_offsets = msg_div_offsets;
-        const ScaleEpilogue<T> epi{base, RELM_MP_DIV_NONE, plan.offsets, nullptr};
-        return run_csr<T, V, G>(plan, op, geo.slices, partial, out, s, epi);
-    });
+        return op;
+    };
+    const ScaleEpilogue<T> epi{base, RELM_MP_DIV_NONE, plan.offsets, nullptr};
+    return run_csr<T>(plan, csr_lanes<T, Reduction::kDivided>(emb, aligned16(table)), emb, partial, out, s, make, epi);
 }
 
 int compute_segment_sum_msgdiv(int dtype, const relm_mp_plan& plan, const void* table, int64_t emb,
@@ -1754,7 +1831,7 @@ int rows_scale_t(const void* in_v, const int64_t* gather, int div_kind, const in
     const T* base = static_cast<const T*>(base_v);
     T* out = static_cast<T*>(out_v);
     const Geometry geo = choose_geometry<T>(emb, out == in || out == base);
-    return with_geometry<T>(geo, [&](auto vt, auto gt) -> int {
+    return with_geometry<T, true>(geo, [&](auto vt, auto gt) -> int {
         constexpr int V = decltype(vt)::value;
         constexpr int G = decltype(gt)::value;
         hipLaunchKernelGGL((k_rows_scale<T, V, G>), row_grid(rows, G, geo.slices, gather_rows_in_flight<T, V>()),
@@ -1861,7 +1938,7 @@ int sum_backward_edges_t(const relm_mp_plan& fwd, const relm_mp_plan_counts* cou
     const GathersSnap rows{fwd.snap_gathers, fwd.snap_gather_plain};
     const GathersSnap dsts{fwd.snap_keys, fwd.snap_key_plain};
     const Geometry geo = choose_geometry<T>(emb);
-    return with_geometry<T>(geo, [&](auto vt, auto gt) -> int {
+    return with_geometry<T, false>(geo, [&](auto vt, auto gt) -> int {
         constexpr int V = decltype(vt)::value;
         constexpr int G = decltype(gt)::value;
         hipLaunchKernelGGL((k_gather_edges<T, V, G>), row_grid(E, G, geo.slices, gather_rows_in_flight<T, V>()),
