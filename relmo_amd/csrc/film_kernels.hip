@@ -322,12 +322,18 @@ int64_t film_rows_per_block(const FilmLayout& L, int64_t rows, int least, int mo
     return static_cast<int64_t>(per_thread) * L.phases;
 }
 
-// 4 floats to a unit, at any alignment; rows narrower than that go one by one,
-// and so do rows whose last unit would share columns with the one before it
-// where the output takes the place of an input: a column must not be read again
-// after another thread has written it.
+// Floats of a unit: 4 at any alignment where they divide the row or the columns
+// that the last unit computes twice are few (from 64 on), else 2.  In units of 4
+// the forward of 67 M floats takes 287 us at width 6 and 252 at 10, the backward 459
+// at 5 and 404 at 6; in units of 2 213, 208, 339 and 308 (227, 238, 407 and 361 by
+// rows of whole 8- or 4-byte lanes in larger workgroups); at 201 and 398 the forward
+// 269 and 238 us against 285 and 243.  3 floats go one by one (backward 305 us, 368
+// in units of 2).  Where the output takes the place of an input, units that share no
+// column: one must not be read again after another thread has written it.
 int film_vec(int64_t width, bool in_place = false) {
-    return width >= 4 && !(in_place && width % 4 != 0) ? 4 : 1;
+    const int V = width % 4 == 0 || width >= 64 ? 4 : width == 1 || width == 3 ? 1 : 2;
+    if (in_place && width % V != 0) return width % 2 == 0 ? 2 : 1;
+    return V;
 }
 
 hipError_t film_backward(const float* s, const float* dy, int64_t width, const FilmRanges& R,
@@ -337,7 +343,9 @@ hipError_t film_backward(const float* s, const float* dy, int64_t width, const F
     const FilmLayout L = film_layout(width, V);
     const dim3 grid(static_cast<unsigned>(R.first_block[kMaxRanges] * L.chunks));
     const size_t lds = static_cast<size_t>(L.phases) * L.units * V * 2 * sizeof(double);
-    const auto kernel = V == 4 ? k_film_mish_backward<4> : k_film_mish_backward<1>;
+    const auto kernel = V == 4   ? k_film_mish_backward<4>
+                        : V == 2 ? k_film_mish_backward<2>
+                                 : k_film_mish_backward<1>;
     hipLaunchKernelGGL(kernel, grid, dim3(kThreads), lds, st, s, dy, width, R, L, gamma, beta, add, ds, partial);
     return hipGetLastError();
 }
@@ -359,7 +367,7 @@ hipError_t launch_film_mish(const float* s, int64_t width, const int64_t* range_
     const FilmLayout L = film_layout(width, V);
     const FilmRanges R = film_ranges(range_start, num_ranges, film_rows_per_block(L, rows, 4, 16));
     const dim3 grid(static_cast<unsigned>(R.first_block[kMaxRanges] * L.chunks));
-    const auto kernel = V == 4 ? k_film_mish<4> : k_film_mish<1>;
+    const auto kernel = V == 4 ? k_film_mish<4> : V == 2 ? k_film_mish<2> : k_film_mish<1>;
     hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, st, s, width, R, L, gamma, beta, add, y);
     return hipGetLastError();
 }

@@ -134,7 +134,10 @@ def test_film_mish_bitwise_against_torch_over_float_ranges(lo_bits: int, hi_bits
 @pytest.mark.parametrize("width,starts", [
     (1, [0, 1]),                       # rows narrower than one unit
     (3, [0, 5, 5, 1300]),
+    (2, [0, 300]),
     (5, [0, 70, 4099]),                # the last unit shares columns with the one before
+    (6, [0, 5, 1300]),                 # units of two floats
+    (63, [0, 129, 1100]),
     (64, [0, 0, 16, 17, 1041]),        # empty and one-row ranges
     (257, [0, 129, 20000]),            # two column chunks, the second shorter
     (400, [0, 33]),
@@ -161,7 +164,7 @@ def test_film_mish_backward_sums(width, starts) -> None:
         b0 += nb
 
 
-@pytest.mark.parametrize("width", [5, 131, 257, 400])  # the last unit shared, over chunks too, and not
+@pytest.mark.parametrize("width", [5, 30, 66, 131, 257, 400])  # the last unit shared, over chunks too, and not
 def test_film_mish_in_place(width: int) -> None:
     """The output over the input (y over s, ds over s or dy): the bits of a call with buffers of its own."""
 
