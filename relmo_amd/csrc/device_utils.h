@@ -50,6 +50,17 @@ __device__ __forceinline__ unsigned long long match_digit(uint32_t digit,
     return (static_cast<unsigned long long>(hi) << 32) | lo;
 }
 
+// Between an LDS store of one lane and the other lanes' reads of it in the same
+// wave, which needs no instruction but has to be said: without it a lane that
+// does not store may keep a value it has read before where the address is the
+// same for all (the radix sort's counts at a digit of no bits), and with a fence
+// alone its next read may be moved into its side of the branch around the store
+// and run before it.  The barrier keeps the lanes together, the fence the memory.
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // V elements of a row as one load / store, at any address aligned to one
 // element: global memory takes 8- and 16-byte accesses at dword alignment.  The
 // elements are spelled out one by one and the compiler joins them: written as

@@ -680,6 +680,7 @@ __global__ __launch_bounds__(kDownThreads) void k_radix_downsweep(
             if (active) before = wcnt[wave][d];
             rank[r] = before + below;
             if (active && below == 0) wcnt[wave][d] = before + __popcll(peers);
+            wave_lds_sync();
         }
     };
     if (tile_base + kSortTile <= n)

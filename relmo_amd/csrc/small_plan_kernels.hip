@@ -166,7 +166,7 @@ __global__ __launch_bounds__(kThreads) void k_csr_small(
                 const uint32_t before = active ? wcnt[wave][d] : 0u;
                 rank[r] = before + below;
                 if (active && below == 0) wcnt[wave][d] = before + __popcll(peers);
-                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                wave_lds_sync();
             }
         }
         __syncthreads();

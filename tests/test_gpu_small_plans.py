@@ -178,3 +178,25 @@ def test_csr_build_reads_no_index_array_after_it_returns(num_keys: int, num_edge
         short = np.repeat(np.diff(offsets) <= bp.plan.hub_threshold, np.diff(offsets))
         assert np.array_equal(_np(bp.short_gather), gathers[perm][short])
         assert capi.plan_match(_t(keys), _t(gathers), [bp]) == [True]
+
+
+@pytest.mark.parametrize("num_edges", [16385, 20480, 100_001])
+def test_one_key_past_the_small_plans(num_edges: int) -> None:
+    """One key and more edges than a small plan takes: a sort by digits of no bits, whose ranks count on through
+    the rounds of a wave (they started again at each round: rows never written, and read by the reduction)."""
+
+    from relmo_amd import capi
+
+    print(f"one key, {num_edges} edges", flush=True)
+    rng = np.random.default_rng(num_edges)
+    kt = torch.zeros(num_edges, dtype=torch.int64, device=DEV)
+    for gathers in (None, np.arange(num_edges), rng.permutation(num_edges)):
+        bp = capi.csr_plan(kt, 1, None if gathers is None else _t(gathers), num_edges)
+        want = np.arange(num_edges) if gathers is None else gathers
+        assert np.array_equal(_np(bp.gather_sorted), want)
+        assert np.array_equal(_np(bp.offsets), [0, num_edges])
+        assert (bp.plan.max_degree, bp.plan.num_hubs) == (num_edges, 1)
+    x = torch.randn(num_edges, 32, device=DEV, generator=torch.Generator(device=DEV).manual_seed(1))
+    got = capi.plan_segment_reduce(bp, x, 0)
+    n = num_edges * torch.finfo(torch.float32).eps
+    assert bool(((got.double() - x.double().sum(0)).abs() <= n * x.double().abs().sum(0)).all())
