@@ -381,7 +381,7 @@ int inv_build(const int64_t* keys, int64_t key_bound, const char* key_name, cons
     plan->snap_gathers = reinterpret_cast<const int32_t*>(snap.gathers);
     plan->snap_gather_plain = snap.gather_plain;
     int32_t gen = 0;
-    if (small_plan(num_edges, key_bound)) {
+    if (small_inv_plan(num_edges, key_bound)) {
         const StatusPublish pub = hs->publish_target(l.status, &gen);
         RELM_HIP(launch_inv_small(keys, key_bound, gathers, gather_bound, num_edges, l.inv, snap,
                                   l.counts, l.status, pub, s),
@@ -485,7 +485,7 @@ int csr_build(const int64_t* keys, int64_t key_bound, const char* key_name, cons
     plan->max_degree = plan->num_hubs = plan->num_chunks = plan->num_multi_hubs = -1;
     plan->num_items = plan->num_short = -1;
     int32_t status_gen = 0;
-    if (small_plan(num_edges, key_bound)) {
+    if (small_csr_plan(num_edges, key_bound)) {
         const StatusPublish pub = hs != nullptr ? hs->publish_target(l.status, &status_gen) : StatusPublish{};
         const SmallCsr small{l.offsets, l.gather_sorted, l.hub_key, l.hub_chunk_base, l.multi_hubs,
                              l.chunk_hub, l.item_first, l.item_short, l.num_items, l.short_off,

@@ -148,9 +148,13 @@ hipError_t launch_key_index(const int32_t* offsets, const int32_t* gather_sorted
                             relm_mp_plan_counts* counts, DevStatus* st, hipStream_t s);
 
 // ---- plans of small inputs (small_plan_kernels.hip) -------------------------
-// Edges and keys that one workgroup's LDS takes.
+// Edges and keys that one workgroup's LDS takes, and edges and keys together up
+// to which its CSR build is the faster one (times of both in launch_csr_small and
+// launch_inv_small).
 constexpr int kSmallPlanMax = 16384;
-bool small_plan(int64_t num_edges, int64_t num_keys);
+constexpr int kSmallCsrMax = 24000;
+bool small_inv_plan(int64_t num_edges, int64_t num_keys);
+bool small_csr_plan(int64_t num_edges, int64_t num_keys);
 // The arrays of a CSR plan (relm_mp_plan), as csr_layout carves them.
 struct SmallCsr {
     int32_t* offsets;
@@ -169,7 +173,8 @@ struct SmallCsr {
     uint32_t* snap_plain;
     relm_mp_plan_counts* counts;
 };
-// The whole build of a plan for which small_plan holds, the status included.
+// The whole build of a plan for which small_csr_plan or small_inv_plan holds, the
+// status included.
 hipError_t launch_csr_small(const int64_t* keys, int64_t key_bound, const int64_t* gathers,
                             int64_t gather_bound, int64_t n, const SmallCsr& a, DevStatus* st,
                             const StatusPublish& pub, hipStream_t s);

@@ -4,10 +4,9 @@
 // launches, an inverse build one of 4; below some ten thousand edges each of
 // them runs for its latency only (2 to 12 us in a few workgroups) and the chain
 // is what the build costs.  Here the whole build stays in the LDS of one
-// workgroup: 3,200 edges over 200 keys take 16 us in one launch instead of 33 us
-// in eight, the inverse map 8 us instead of 19 us in four.  The work grows with
-// the edges on one compute unit while the chain's latency does not, so inputs
-// past kSmallPlanMax edges or keys go to the general kernels.
+// workgroup.  The work grows with the edges and keys on one compute unit while
+// the chain's latency does not, so larger inputs go to the general kernels
+// (small_csr_plan, small_inv_plan).
 //
 // The plans are those of the general kernels, array for array; only the
 // snapshot tiles flagged plain are stored here too (nothing reads them).
@@ -204,7 +203,9 @@ __global__ __launch_bounds__(kThreads) void k_csr_small(
         if (p + 1 == n || sk[p + 1] >> kPosBits != k) sx[k] = static_cast<uint32_t>(p) + 1u;
     }
     __syncthreads();
-    const int kpt = nk / kThreads + 1;  // consecutive keys per thread, key nk (the end) among them
+    // consecutive keys per thread, key nk (the end) among them: an odd number, so
+    // that the threads of a wave, which read kpt apart, hit different banks
+    const int kpt = (nk / kThreads + 1) | 1;
     const int k0 = min(tid * kpt, nk + 1), k1 = min(k0 + kpt, nk + 1);
     uint32_t last = 0;
     for (int k = k0; k < k1; ++k) last = max(last, sx[k]);
@@ -370,10 +371,18 @@ __global__ __launch_bounds__(kThreads) void k_inv_small(
 
 }  // namespace
 
-bool small_plan(int64_t num_edges, int64_t num_keys) {
+bool small_inv_plan(int64_t num_edges, int64_t num_keys) {
     return num_edges > 0 && num_edges <= kSmallPlanMax && num_keys <= kSmallPlanMax;
 }
 
+bool small_csr_plan(int64_t num_edges, int64_t num_keys) {
+    return small_inv_plan(num_edges, num_keys) && num_edges + num_keys <= kSmallCsrMax;
+}
+
+// Builds back to back, here and by the general kernels: 3,200 edges over 200 keys
+// 15 and 35 us, 8,192 over 8,192 32 and 44, 16,384 over 1,000 39 and 41, over 7,500
+// 45 and 45, over 16,384 56 and 45; 12,288 over 12,288 44 and 45, over 15,500 49 and
+// 45; 8,192 over 16,384 43 and 46.
 hipError_t launch_csr_small(const int64_t* keys, int64_t key_bound, const int64_t* gathers,
                             int64_t gather_bound, int64_t n, const SmallCsr& a, DevStatus* st,
                             const StatusPublish& pub, hipStream_t s) {
@@ -385,6 +394,9 @@ hipError_t launch_csr_small(const int64_t* keys, int64_t key_bound, const int64_
     return hipGetLastError();
 }
 
+// Builds back to back, here and by the general kernels: 3,200 edges over 200 keys
+// 16 and 25 us, 8,192 over 8,192 20 and 32, 16,384 over 16,384 25 and 33: the limit
+// is the LDS.
 hipError_t launch_inv_small(const int64_t* keys, int64_t key_bound, const int64_t* gathers,
                             int64_t gather_bound, int64_t n, int32_t* inv, const SnapOut& snap,
                             relm_mp_plan_counts* counts, DevStatus* st, const StatusPublish& pub,

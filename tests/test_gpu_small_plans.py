@@ -200,3 +200,12 @@ def test_one_key_past_the_small_plans(num_edges: int) -> None:
     got = capi.plan_segment_reduce(bp, x, 0)
     n = num_edges * torch.finfo(torch.float32).eps
     assert bool(((got.double() - x.double().sum(0)).abs() <= n * x.double().abs().sum(0)).all())
+
+
+@pytest.mark.parametrize("num_keys,num_edges", [(7616, 16384), (7617, 16384), (16384, 7616), (15360, 4097), (11999, 12001)])
+@pytest.mark.parametrize("form", ["permuted", "skewed"])
+def test_small_plans_at_the_limit_of_edges_and_keys(num_keys: int, num_edges: int, form: str) -> None:
+    """Up to and past the sum of edges and keys that one workgroup's CSR build takes, even numbers of keys per
+    thread among them."""
+
+    test_small_plans_against_the_oracle(num_keys, num_edges, form)
