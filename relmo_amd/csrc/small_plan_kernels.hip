@@ -36,9 +36,7 @@ __device__ __forceinline__ void publish(const DevStatus& v, DevStatus* __restric
     *st = v;
     if (pub.host == nullptr) return;
     *pub.host = v;
-    __threadfence_system();
-    if (pub.host_gen != nullptr)
-        __hip_atomic_store(pub.host_gen, pub.gen, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    __hip_atomic_store(pub.host_gen, pub.gen, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 __device__ __forceinline__ DevStatus new_status(uint32_t bad_key, uint32_t bad_gather) {
@@ -356,8 +354,8 @@ __global__ __launch_bounds__(kThreads) void k_inv_small(
     }
     // Published behind the whole plan, as by the general build: the host's word
     // is all that a caller waits for before other streams read the map or its
-    // memory is used again.  Every wave releases its own stores first.
-    __threadfence();
+    // memory is used again.  The barrier orders the workgroup's stores before the
+    // publishing thread's system-scope release, which covers them all.
     __syncthreads();
     if (tid == 0) {
         DevStatus v = new_status(s_bad[0], s_bad[1]);
