@@ -339,8 +339,8 @@ int relm_mp_plan_fanin_backward_by_dst(int dtype, const relm_mp_plan* dst_plan,
  * (that call's work on `stream` precedes this one); only the backward kernel is
  * launched, without waiting, and *collisions is 0.  With rel_rows ==
  * num_edges the map is built without an initial fill (an injective flat_src
- * writes every row) and the sum (mode 0) runs in edge order over the plan's
- * snapshots, each edge writing its own row.  No reference counterpart:
+ * writes every row) and the sum (mode 0) over rows of whole 16-byte units runs in
+ * edge order over the plan's snapshots, each edge writing its own row.  No reference counterpart:
  * it replaces the inverse-plan build of the backward ops (mp_ops.cpp:3224-3325
  * take flat_src and dst_idx afresh) for callers that hold the forward's plan. */
 int relm_mp_plan_fanin_backward_by_src(int dtype, const relm_mp_plan* dst_plan, int64_t mode,

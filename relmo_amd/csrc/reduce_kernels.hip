@@ -1978,8 +1978,8 @@ int compute_backward_by_src(int dtype, const relm_mp_plan& dst_plan, const relm_
         const size_t ib = static_cast<size_t>(dst_plan.num_edges) * sizeof(int32_t);
         if (tb + ib <= kPrefetchMaxBytes && tb % 16 == 0 && ib % 16 == 0 &&
             (reinterpret_cast<uintptr_t>(grad_out) | reinterpret_cast<uintptr_t>(dst_plan.snap_keys)) % 16 == 0) {
-            const int64_t units = static_cast<int64_t>((tb + ib) / 16);
-            const int64_t blocks = std::min<int64_t>((units + kThreads * 8 - 1) / (kThreads * 8), 4096);
+            const int64_t words = static_cast<int64_t>((tb + ib) / 16);
+            const int64_t blocks = std::min<int64_t>((words + kThreads * 8 - 1) / (kThreads * 8), 4096);
             hipLaunchKernelGGL(k_touch, dim3(static_cast<unsigned>(std::max<int64_t>(blocks, 1))),
                                dim3(kThreads), 0, s, static_cast<const uint4*>(grad_out),
                                static_cast<int64_t>(tb / 16), reinterpret_cast<const uint4*>(dst_plan.snap_keys),
