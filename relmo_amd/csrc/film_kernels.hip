@@ -68,8 +68,7 @@ __device__ __forceinline__ float mish_backward(float dy, float u) {
 }
 
 // V floats that start at any 4-byte aligned address: one 16-byte access for V =
-// 4 (global memory takes it at dword alignment), so rows of any width move in
-// 16-byte pieces.
+// 4, one of 8 for V = 2 (global memory takes them at dword alignment).
 template <int V>
 using Vec = float __attribute__((ext_vector_type(V), aligned(4)));
 
@@ -140,9 +139,9 @@ __device__ __forceinline__ FilmThread film_thread(const FilmLayout& L, int chunk
 // first of them is used.
 constexpr int kRows = 2;
 
-// Bound by the vector units, not by memory: about 125 lane instructions per
-// element, three quarters of them log1pf, so 400 M elements take 1.2 ms at any
-// split while moving them takes 0.64.  The workgroups are small (4 waves) and
+// Bound by the vector units, not by memory: 160 lane instructions per element
+// (counted; most of them in expf, log1pf and tanhf), so 400 M elements take 1.2 ms
+// at any split while moving them takes 0.64.  The workgroups are small (4 waves) and
 // many, so that the last ones leave few CUs idle: [1,000,003 x 400] takes 1.34
 // ms, [204,800 x 96] 76 us and [2,000 x 400] 10 us, against 1.46 ms, 86 us and
 // 158 us with 768 threads to a workgroup of 512 whole rows.
@@ -183,7 +182,8 @@ __global__ __launch_bounds__(kThreads) void k_film_mish(const float* __restrict_
 // its rows in row order, then the phases in order.  The block sums stay fp64
 // (a range's blocks are added in fp64 and rounded once), so a per-range sum
 // over tens of thousands of rows carries only the rounding of its terms.
-// `lds` holds phases * units * V * 2 doubles.  Bound as the forward is: [1,000,003
+// `lds` holds phases * units * V * 2 doubles.  Bound as the forward is (195 lane
+// instructions per element): [1,000,003
 // x 400] takes 1.67 ms with the sums, [204,800 x 96] 101 us, against 2.18 ms and
 // 134 us with the forward's former split and torch's sums.
 template <int V>

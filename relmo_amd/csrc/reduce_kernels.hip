@@ -1,10 +1,11 @@
 // Row kernels of the relational message-passing ops.
 //
 // Every output row is owned by exactly one "row group" of G lanes (G = 4..64,
-// a divisor of the wave), each lane moving V contiguous elements (16 bytes;
-// one element where a row is narrower than that) at any alignment; rows wider
-// than G*V are split over blockIdx.y slices.  No atomics anywhere: the messages of a key are visited
-// in the stable (edge) order of the plan, so every result is deterministic.
+// a divisor of the wave), each lane moving V contiguous elements at any
+// alignment (16 bytes, or fewer where that is faster: choose_geometry,
+// csr_lanes); rows wider than G*V are split over blockIdx.y slices.  No atomics
+// anywhere: the messages of a key are visited in the stable (edge) order of the
+// plan, so every result is deterministic.
 //
 // CSR plans are reduced in two parts:
 //  * segments of at most kHubThreshold messages: k_walk_items.  Key k weighs
@@ -51,7 +52,6 @@ constexpr size_t kPrefetchMaxBytes = size_t(256) << 20;
 // row.  Where V does not divide D the row's last lane is moved back to end with
 // the row; the columns it shares with the lane before are computed twice, with
 // equal results (each column's values and order do not depend on the lane).
-// Rows of 33 floats so take 9 lanes of a group of 16 instead of 33 lanes of 64.
 template <int V, int G>
 __device__ __forceinline__ uint32_t lane_column(int gl, int64_t D) {
     const uint32_t c = blockIdx.y * (G * V) + static_cast<uint32_t>(gl) * V;
